@@ -195,19 +195,25 @@ def paged_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_le
     block_tables: [B, max_blocks_per_seq] int32, physical block ids
     context_lens: [B] int32, tokens of context per sequence (>= 1)
     max_context_len: Python int, max(context_lens) (passed in to avoid a sync)
-    partition_size: tokens per split (multiple of 256). None picks one from the
-                  batch size; a value >= max_context_len disables split-K.
+    partition_size: tokens per split (multiple of 256); a value >= max_context_len
+                  disables split-K.  None: the kernel cuts the contexts into splits
+                  of about equal size; where it does not (one sequence, more than
+                  64, contexts up to 1024 tokens), decode_partition picks one.
     """
     if not (q.dtype == k_cache.dtype == v_cache.dtype == torch.float16):
         raise ValueError("q and caches must be fp16")
     if q.shape[-1] not in (64, 128) or k_cache.shape[-1] != q.shape[-1]:
         raise ValueError("head_dim must be 64 or 128 and match the cache")
     scale = 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale
+    ext = load_extension()
     if partition_size is None:
+        run = ext.paged_decode_balanced
         partition_size = decode_partition(q.shape[0], k_cache.shape[1], max_context_len,
                                           q.device.index)
+    else:
+        run = ext.paged_decode
     partition_size = -(-int(partition_size) // CHUNK) * CHUNK
-    return load_extension().paged_decode(
+    return run(
         q.contiguous(), k_cache.contiguous(), v_cache.contiguous(),
         block_tables.to(torch.int32).contiguous(), context_lens.to(torch.int32).contiguous(),
         int(max_context_len), float(scale), partition_size)

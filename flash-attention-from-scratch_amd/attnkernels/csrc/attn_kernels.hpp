@@ -48,6 +48,12 @@ struct DecodeArgs {
     int32_t* counters;
     int64_t batch, hq, hkv, d, num_blocks, bs, max_blocks;
     int64_t partition, num_splits;
+    // Balanced splits: the kernels cut the sequences themselves, from the
+    // context lengths they find (each at most token_cap), into at most
+    // num_splits splits per kv head, of `partition` tokens or more; counters
+    // are set, and the partials are [hq, num_splits] rows.
+    bool balanced = false;
+    int64_t token_cap = 0;
     float sl2;             // scale * log2(e)
     void* stream;
 };
@@ -65,6 +71,16 @@ struct CacheWriteArgs {
 
 hipError_t prefill_launch(const PrefillArgs& a);
 hipError_t decode_launch(const DecodeArgs& a);
+
+// Balanced splits: most sequences (one lane of a wave each), and the fewest
+// tokens worth a split of their own (256: one iteration of an 8-wave
+// matrix-core workgroup; at 512 short contexts lost 0.4-1 us, at 128 they
+// gained nothing).
+constexpr int64_t kBalancedMaxBatch = 64;
+constexpr int64_t kBalancedMinSplit = 256;
+// Workgroups per kv head of a balanced launch for these sizes (max_ctx: the
+// longest context, cap: the most tokens read of one), 0: use fixed splits.
+int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap);
 
 // Size of the static per-GPU split-partials array behind
 // ak_paged_decode_noalloc, and its device address on the current GPU

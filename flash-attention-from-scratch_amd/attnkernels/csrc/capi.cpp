@@ -1,6 +1,7 @@
 // C-ABI entry points (include/attnkernels.h): argument validation, the
 // reference's error wording, and dispatch to the HIP launchers.  Validation
 // runs before any HIP call, so a rejected call never touches the GPU.
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -133,12 +134,23 @@ size_t partials_bytes(int64_t batch, int64_t num_heads, int64_t splits, int64_t 
     return (size_t)batch * (size_t)num_heads * (size_t)splits * (size_t)(head_dim + 2) * sizeof(float);
 }
 
-void set_partials(ak::DecodeArgs& a, void* buf) {
+void set_partials(ak::DecodeArgs& a, void* buf, size_t rows) {
     float* ws = static_cast<float*>(buf);
-    const size_t rows = (size_t)a.batch * (size_t)a.hq * (size_t)a.num_splits;
     a.o_part = ws;
     a.m_part = ws + rows * (size_t)a.d;
     a.l_part = a.m_part + rows;
+}
+
+// Workgroups per kv head of the balanced launch for these sizes; 0: none
+// (invalid sizes, or fixed splits serve).  The most tokens it reads of a
+// sequence are those fixed splits of `partition` tokens would read.
+int64_t balanced_workers(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                         int64_t max_context_len, int64_t partition) {
+    if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 || head_dim <= 0 || partition <= 0 ||
+        max_context_len < 1 || max_context_len > INT_MAX - partition)
+        return 0;
+    const int64_t cap = (max_context_len + partition - 1) / partition * partition;
+    return ak::decode_balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len, cap);
 }
 
 }  // namespace
@@ -235,10 +247,50 @@ int ak_paged_decode_fused(const void* q, const void* k_cache, const void* v_cach
                                               " bytes required, got " + std::to_string(workspace_bytes));
         if (!aligned16(workspace))
             return fail(AK_ERR_INVALID_ARGUMENT, "paged_decode: workspace must be 16-byte aligned");
-        set_partials(a, workspace);
+        set_partials(a, workspace, (size_t)(a.batch * a.hq * a.num_splits));
         a.counters = counters;
     }
     return hip_status(ak::decode_launch(a), "paged_decode");
+}
+
+size_t ak_paged_decode_balanced_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                               int64_t head_dim, int64_t max_context_len, int64_t partition) {
+    return partials_bytes(1, num_heads, balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len,
+                                                         partition), head_dim);
+}
+
+int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
+                             const int32_t* context_lens, void* out, int64_t batch, int64_t num_heads,
+                             int64_t num_kv_heads, int64_t head_dim, int64_t num_blocks, int64_t block_size,
+                             int64_t max_blocks_per_seq, int64_t max_context_len, double scale, int64_t partition,
+                             void* workspace, size_t workspace_bytes, int32_t* counters, int64_t counters_len,
+                             void* stream) {
+    ak::DecodeArgs a{};
+    const int rc = decode_args(q, k_cache, v_cache, block_tables, context_lens, out, batch, num_heads, num_kv_heads,
+                               head_dim, num_blocks, block_size, max_blocks_per_seq, max_context_len, scale,
+                               partition, stream, a);
+    if (rc != AK_OK || batch == 0) return rc;
+    const int64_t workers = balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len, partition);
+    if (workers == 0)
+        return fail(AK_ERR_UNSUPPORTED, "paged_decode_balanced: fixed splits serve these sizes "
+                                        "(ak_paged_decode_balanced_workspace_size is 0)");
+    if (!counters || counters_len < batch * num_kv_heads || (reinterpret_cast<uintptr_t>(counters) & 3u))
+        return fail(AK_ERR_INVALID_ARGUMENT, "paged_decode_balanced: counters must be a 4-byte aligned int32 array of "
+                                             "at least batch * num_kv_heads = " +
+                                                 std::to_string(batch * num_kv_heads) + " elements");
+    const size_t need = partials_bytes(1, num_heads, workers, head_dim);
+    if (!workspace || workspace_bytes < need)
+        return fail(AK_ERR_WORKSPACE, "paged_decode_balanced: workspace of " + std::to_string(need) +
+                                          " bytes required, got " + std::to_string(workspace_bytes));
+    if (!aligned16(workspace))
+        return fail(AK_ERR_INVALID_ARGUMENT, "paged_decode_balanced: workspace must be 16-byte aligned");
+    a.token_cap = std::min(a.num_splits * a.partition, a.max_blocks * a.bs);
+    a.balanced = true;
+    a.partition = ak::kBalancedMinSplit;
+    a.num_splits = workers;
+    a.counters = counters;
+    set_partials(a, workspace, (size_t)a.hq * (size_t)workers);
+    return hip_status(ak::decode_launch(a), "paged_decode_balanced");
 }
 
 int ak_paged_decode_noalloc(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
@@ -273,7 +325,7 @@ int ak_paged_decode_noalloc(const void* q, const void* k_cache, const void* v_ca
         int32_t* counters = nullptr;
         const hipError_t e = ak::decode_scratch(&ws, &counters);
         if (e != hipSuccess) return hip_status(e, "paged_decode_noalloc");
-        set_partials(a, ws);
+        set_partials(a, ws, (size_t)(a.batch * a.hq * a.num_splits));
         // counters for every (sequence, kv head) fit the static array: merged in
         // the decode kernel; otherwise by the reduce kernel
         if ((size_t)batch * (size_t)num_kv_heads <= ak::kDecodeScratchCounters) a.counters = counters;

@@ -61,7 +61,7 @@ __device__ __forceinline__ f32x4 coherent_load4(const float* p) {  // 16-byte al
 // SG split groups of a unit are merged through LDS.
 template <int D, int G, int THREADS>
 __device__ __forceinline__ void merge_splits(const float* o_part, const float* m_part, const float* l_part,
-                                             f16* out, size_t row0, int num_splits, int ns, int tid) {
+                                             f16* out, size_t row0, size_t slot0, size_t hstride, int ns, int tid) {
     // NB: loads per batch, enough for the most splits merged here in one batch,
     // but no more than the kernel's main loop has registers for (8, or 16 for
     // the four- and eight-head kernels)
@@ -73,10 +73,10 @@ __device__ __forceinline__ void merge_splits(const float* o_part, const float* m
     __shared__ f32x4 mg_o[THREADS];
     const int u = tid % UNITS, sg = tid / UNITS;
     const int h = u / (D / 4), d4 = u % (D / 4);
-    const size_t row = row0 + h;
-    const float* mp = m_part + row * num_splits;
-    const float* lp = l_part + row * num_splits;
-    const float* op = o_part + row * num_splits * D + d4 * 4;
+    const size_t row = row0 + h, slot = slot0 + h * hstride;
+    const float* mp = m_part + slot;
+    const float* lp = l_part + slot;
+    const float* op = o_part + slot * D + d4 * 4;
     float M = -INFINITY, L = 0.f;
     f32x4 O = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = sg; s0 < ns; s0 += SG * NB) {
@@ -133,6 +133,98 @@ __device__ __forceinline__ void merge_splits(const float* o_part, const float* m
     }
 }
 
+// The work of one workgroup: tokens [start, end) of sequence b, the split-th of
+// the ns splits of that sequence that hold tokens, and where its partials go:
+// head h of the kv head's group at index slot0 + h * hstride + split.  b < 0:
+// nothing to do.
+struct Segment {
+    int b, split, ns, start, end;
+    size_t slot0, hstride;
+};
+
+// Splits of a fixed number of tokens (grid: kv head, split, sequence).
+__device__ __forceinline__ Segment fixed_segment(const int* __restrict__ ctx_lens, int h0, int hq, int max_tok,
+                                                 int partition, int num_splits) {
+    Segment sg;
+    sg.b = blockIdx.z;
+    sg.split = blockIdx.y;
+    const int ctx = min(ctx_lens[sg.b], max_tok);
+    sg.start = sg.split * partition;
+    sg.end = min(ctx, sg.start + partition);
+    const int ns = ctx > 0 ? (int)(((long long)ctx + partition - 1) / partition) : 0;
+    sg.ns = min(ns, num_splits);  // the reduce kernel reads as many
+    sg.slot0 = ((size_t)sg.b * hq + h0) * num_splits;
+    sg.hstride = num_splits;
+    return sg;
+}
+
+// Inclusive sum over the lanes of a wave (DPP row shifts, then row broadcasts).
+__device__ __forceinline__ int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);   // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);   // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);   // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
+// Splits of about equal size, cut from the context lengths the kernel finds:
+// grid (kv head, workgroup), `workers` workgroups per kv head, one split each.
+// A fixed partition gives a ragged batch workgroups of very different
+// lengths, and most of the grid may be empty; HBM then idles while the longest
+// ones finish.  Here every wave reads all the lengths (one load, a lane per
+// sequence), looks for the smallest split size (at least min_split tokens, a
+// multiple of GRAN, the tokens of one workgroup iteration) for which the
+// sequences have at most `workers` splits in all, and cuts each sequence into
+// that many even ones.  Every workgroup of every kv head finds the same cut.
+template <int G, int GRAN>
+__device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_lens, int kvh, int min_split,
+                                                    int workers, int batch, int cap, int lane) {
+    const int c = lane < batch ? min(max(ctx_lens[lane], 0), cap) : -1;
+    const int total = __builtin_amdgcn_readlane(wave_scan(max(c, 0)), 63);
+    auto round_up = [](int x) { return (x + GRAN - 1) / GRAN * GRAN; };
+    // No smaller size can do; even batches take this one.
+    int size = max(min_split, round_up(1 + (int)((float)(total - 1) * __builtin_amdgcn_rcpf((float)workers))));
+    int n, incl;
+    for (int it = 0;; ++it) {
+        // ceil(c / size), a float quotient put right by one step either way
+        // (c < 2^24), at least 1 (an empty sequence's workgroup writes its zero rows).
+        n = (int)((float)c * __builtin_amdgcn_rcpf((float)size));
+        n += n * size < c ? 1 : 0;
+        n -= (n - 1) * size >= c ? 1 : 0;
+        n = c < 0 ? 0 : max(1, n);
+        incl = wave_scan(n);
+        const int count = __builtin_amdgcn_readlane(incl, 63);
+        if (count <= workers) break;
+        size = it < 6 ? round_up(size + 1 + (int)((float)size * (float)(count - workers) *
+                                                  __builtin_amdgcn_rcpf((float)workers)))
+                      : round_up(cap);  // one split per sequence: batch <= workers
+    }
+    const int j = blockIdx.y;
+    Segment sg;
+    sg.b = -1;
+    sg.split = sg.ns = sg.start = sg.end = 0;
+    sg.slot0 = 0;
+    sg.hstride = workers;
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(j >= incl - n && j < incl);
+    if (hit) {
+        const int l = (int)__builtin_ctzll(hit);
+        const int ctx = __builtin_amdgcn_readlane(c, l), ns = __builtin_amdgcn_readlane(n, l);
+        const int base = __builtin_amdgcn_readlane(incl, l) - ns;
+        // Even splits of a multiple of GRAN tokens.  Each holds a token: len <=
+        // size because size is such a multiple, and (ns - 1) * size < ctx.
+        const int len = round_up((int)(((unsigned)ctx + ns - 1) / (unsigned)ns));
+        sg.b = l;
+        sg.split = j - base;
+        sg.ns = ns;
+        sg.start = sg.split * len;
+        sg.end = min(ctx, sg.start + len);
+        sg.slot0 = (size_t)kvh * G * workers + base;
+    }
+    return sg;
+}
+
 // Split epilogue of both decode kernels.  red_acc / red_m / red_l hold the
 // workgroup's per-wave (acc, m, l) of the kv head's G query heads (m in the
 // log2 domain; the stored l is L * lscale).  The waves are merged by the LSE
@@ -150,11 +242,11 @@ template <int D, int G, int NW>
 __device__ __forceinline__ void split_epilogue(const float (&red_acc)[NW][G][D], const float (&red_m)[NW][G],
                                                const float (&red_l)[NW][G], float lscale, f16* __restrict__ out,
                                                float* __restrict__ o_part, float* __restrict__ m_part,
-                                               float* __restrict__ l_part, int32_t* __restrict__ counters, int b,
-                                               int kvh, int hkv, int split, int num_splits, int ns, int tid) {
+                                               float* __restrict__ l_part, int32_t* __restrict__ counters,
+                                               int kvh, int hkv, const Segment& sg, int num_splits, int tid) {
     constexpr int THREADS = NW * kWave;
     __shared__ int last;
-    const int hq = hkv * G;
+    const int hq = hkv * G, b = sg.b, ns = sg.ns;
     const bool direct = num_splits == 1 || (counters && ns == 1);
     const bool fused = counters && !direct;
     for (int idx = tid; idx < G * D; idx += THREADS) {
@@ -176,7 +268,7 @@ __device__ __forceinline__ void split_epilogue(const float (&red_acc)[NW][G][D],
         }
         o = L > 0.f ? o / L : 0.f;
         const size_t row = (size_t)b * hq + kvh * G + h;
-        const size_t slot = row * num_splits + split;
+        const size_t slot = sg.slot0 + (size_t)h * sg.hstride + sg.split;
         if (direct) {
             out[row * D + d] = (f16)o;
         } else if (!fused) {
@@ -200,14 +292,9 @@ __device__ __forceinline__ void split_epilogue(const float (&red_acc)[NW][G][D],
     if (tid == 0) last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ns - 1;
     __syncthreads();
     if (!last) return;
-    merge_splits<D, G, THREADS>(o_part, m_part, l_part, out, (size_t)b * hq + (size_t)kvh * G, num_splits, ns, tid);
+    merge_splits<D, G, THREADS>(o_part, m_part, l_part, out, (size_t)b * hq + (size_t)kvh * G, sg.slot0, sg.hstride, ns,
+                                tid);
     if (tid == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Splits of sequence b that hold tokens (the reduce kernel reads as many).
-__device__ __forceinline__ int splits_with_tokens(int ctx, int partition, int num_splits) {
-    const int ns = ctx > 0 ? (int)(((long long)ctx + partition - 1) / partition) : 0;
-    return min(ns, num_splits);
 }
 
 // One query head per kv head (the reference's decode configurations).
@@ -238,7 +325,8 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
                     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
                     f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                     float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs, int bs_shift,
-                    int max_blocks, int num_blocks, int partition, int num_splits, float sl2) {
+                    int max_blocks, int num_blocks, int partition, int num_splits, float sl2, int balanced, int batch,
+                    int cap) {
     using T = DecodeTile<D>;
     constexpr int G = 1;
     __shared__ float red_acc[T::NW][G][D];
@@ -246,13 +334,16 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
 
     // kv head fastest: neighbouring workgroups read neighbouring 4 KB head
     // blocks of the same pages.
-    const int kvh = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
+    const int kvh = blockIdx.x;
     const int hq = hkv * G;
-    const int start = split * partition;
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
-    const int* bt = block_tables + (size_t)b * max_blocks;
     const int max_tok = max_blocks * bs;  // never index past the table row
+    const Segment sg = balanced ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+                                : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
+    const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
+    if (b < 0) return;
+    const int* bt = block_tables + (size_t)b * max_blocks;
 
     // Page ids of this lane's tokens in the chunk starting at t0, for tokens
     // below lim (-1 elsewhere).  They are loaded one chunk ahead, behind the
@@ -270,19 +361,16 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
     // vector loads of its page ids, which would hold its slot for a vector
     // round trip (measured: a skewed batch's step 12% faster, cfg4 and cfg5
     // unchanged).  The page ids and q follow the check.
-    const int ctx_raw = ctx_lens[b];
     const int stride = T::NW * T::TOK;
     int pg[T::U];
 
-    const int ctx = min(ctx_raw, max_tok);
-    if (start >= ctx) {  // whole workgroup: this split is past the context
+    if (start >= end) {  // whole workgroup: this split is past the context
         // A sequence with no context (outside the >= 1 contract) gets a zero row,
         // as the reduce gives it when there are several splits.
         if (num_splits == 1 || (counters && split == 0))
             for (int idx = tid; idx < D; idx += T::THREADS) out[((size_t)b * hq + kvh) * D + idx] = (f16)0.f;
         return;
     }
-    const int end = min(ctx, start + partition);
     load_pages(start + w * T::TOK, end, pg);
     // q of this head, raw fp16 (scaled after the dot product)
     const f16x8 qv = *reinterpret_cast<const f16x8*>(q + ((size_t)b * hq + kvh) * D + li * 8);
@@ -365,8 +453,8 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
         }
     }
     __syncthreads();
-    split_epilogue<D, G, T::NW>(red_acc, red_m, red_l, 1.f, out, o_part, m_part, l_part, counters, b, kvh, hkv,
-                                split, num_splits, splits_with_tokens(ctx, partition, num_splits), tid);
+    split_epilogue<D, G, T::NW>(red_acc, red_m, red_l, 1.f, out, o_part, m_part, l_part, counters, kvh, hkv, sg,
+                                num_splits, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -513,7 +601,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
                         f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                         float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                         int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits, float sl2,
-                        int balance) {
+                        int balance, int balanced, int batch, int cap) {
     using T = GqaTile<D, G, NW>;
     constexpr int U = T::U, N = T::N, S = T::S, LB = T::LB;
     // P = 2^(s - m + kPShift): the largest P the fast path accepts is 2^kPMax.
@@ -521,13 +609,16 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     __shared__ float red_acc[T::NW][G][D];
     __shared__ float red_m[T::NW][G], red_l[T::NW][G];
 
-    const int kvh = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
+    const int kvh = blockIdx.x;
     const int hq = hkv * G;
-    const int start = split * partition;
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
-    const int* bt = block_tables + (size_t)b * max_blocks;
     const int max_tok = max_blocks * bs;
+    const Segment sg = balanced ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+                                : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
+    const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
+    if (b < 0) return;
+    const int* bt = block_tables + (size_t)b * max_blocks;
 
     // Value index of a partial dot product: j = (slot >> 1) * 2G + head * 2 +
     // (slot & 1).  Stage s of the butterfly resolves bit N >> (s + 1), top
@@ -554,25 +645,22 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
             pg[u] = t < lim ? bt[pi] : -1;
         }
     };
-    const int ctx_raw = ctx_lens[b];
     const int stride = T::NW * T::TOK;
     int pg[U];
     const bool fast_bs = bs == T::TOK;
 
-    const int ctx = min(ctx_raw, max_tok);
-    if (start >= ctx) {
+    if (start >= end) {
         if (num_splits == 1 || (counters && split == 0))
             for (int idx = tid; idx < G * D; idx += T::THREADS)
                 out[((size_t)b * hq + kvh * G + idx / D) * D + idx % D] = (f16)0.f;
         return;
     }
-    const int end = min(ctx, start + partition);
     // The first page id and q after the context check: a workgroup past a
     // short context exits after its one scalar load (the check's wait would
     // also wait for a page id loaded beside it; a skewed batch's step 3%
     // faster, uniform batches unchanged).
     int spg = 0;
-    if (fast_bs && start + w * T::TOK + T::TOK <= min(start + partition, max_tok))
+    if (fast_bs && start + w * T::TOK + T::TOK <= end)
         spg = bt[uniform((start + w * T::TOK) >> 4)];
     f16x8 qv[G];  // register a: query head a ^ fh
 #pragma unroll
@@ -797,8 +885,8 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     __syncthreads();
     // m in the log2 domain of the scores: the kPShift on P cancels in o and is
     // taken out of l here.
-    split_epilogue<D, G, T::NW>(red_acc, red_m, red_l, 1.f / 128.f, out, o_part, m_part, l_part, counters, b, kvh,
-                                hkv, split, num_splits, splits_with_tokens(ctx, partition, num_splits), tid);
+    split_epilogue<D, G, T::NW>(red_acc, red_m, red_l, 1.f / 128.f, out, o_part, m_part, l_part, counters, kvh, hkv,
+                                sg, num_splits, tid);
 }
 
 // Eight query heads per kv head on the matrix cores
@@ -849,7 +937,7 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
                              f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                              float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                              int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits,
-                             float sl2, int balance) {
+                             float sl2, int balance, int balanced, int batch, int cap) {
     using T = GqaMfmaTile<D, G, NW>;
     constexpr int KS = T::KS, DPL = T::DPL;
     typedef _Float16 vrow_t __attribute__((ext_vector_type(DPL)));
@@ -858,33 +946,33 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     __shared__ float red_acc[NW][G][D];
     __shared__ float red_m[NW][G], red_l[NW][G];
 
-    const int kvh = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
+    const int kvh = blockIdx.x;
     const int hq = hkv * G;
-    const int start = split * partition;
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
-    const int* bt = block_tables + (size_t)b * max_blocks;
     const int max_tok = max_blocks * bs;
-    const int ctx_raw = ctx_lens[b];
+    const Segment sg = balanced ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+                                : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
+    const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
+    if (b < 0) return;
+    const int* bt = block_tables + (size_t)b * max_blocks;
     const int stride = NW * T::TOK;
     const bool fast_bs = bs == 16;
     int t0 = start + w * T::TOK;
 
-    const int ctx = min(ctx_raw, max_tok);
-    if (start >= ctx) {
+    if (start >= end) {
         if (num_splits == 1 || (counters && split == 0))
             for (int idx = tid; idx < G * D; idx += T::THREADS)
                 out[((size_t)b * hq + kvh * G + idx / D) * D + idx % D] = (f16)0.f;
         return;
     }
-    const int end = min(ctx, start + partition);
     // The first pair's page ids and the Q^T fragments after the context
     // check, so that a workgroup past a short context (most of a skewed
     // batch's grid) exits after its one scalar load.
     int spa = -1, spb = -1;  // page ids of the pair at t0 (wave-uniform), loaded one pair ahead
-    if (fast_bs && t0 + T::TOK <= min(start + partition, max_tok)) {
+    if (fast_bs && t0 < end) {
         spa = bt[uniform(t0 >> 4)];
-        spb = bt[uniform((t0 >> 4) + 1)];
+        spb = t0 + 16 < end ? bt[uniform((t0 >> 4) + 1)] : -1;
     }
 
     // Q^T fragments: head n (zeros for n >= G), dims 32 s + 8 g .. +7.
@@ -1097,8 +1185,8 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
             for (int j = 0; j < DPL; ++j) red_acc[w][h][DPL * n + j] = acc[j][r];
     }
     __syncthreads();
-    split_epilogue<D, G, NW>(red_acc, red_m, red_l, 1.f / 128.f, out, o_part, m_part, l_part, counters, b, kvh,
-                             hkv, split, num_splits, splits_with_tokens(ctx, partition, num_splits), tid);
+    split_epilogue<D, G, NW>(red_acc, red_m, red_l, 1.f / 128.f, out, o_part, m_part, l_part, counters, kvh, hkv, sg,
+                             num_splits, tid);
 }
 
 // LSE merge of the split partials (paged_decode.cu:204-215): one 256-thread
@@ -1175,23 +1263,6 @@ paged_reduce_kernel(const float* __restrict__ o_part, const float* __restrict__ 
 // from it: -1% to +1%.)
 constexpr bool gqa_pipelined(int d, int g) { return d == 64 && g >= 4; }
 
-// Waves per workgroup of both grouped-query kernels.  A dot-product wave
-// reads one 16-token page per round trip to memory, so a split of P tokens
-// costs P / (16 NW) dependent round trips; with many workgroups per CU they
-// overlap, but in a small grid (one sequence, few kv heads) they are the
-// kernel's critical path.  Measured on MI355X (one call after a 512 MiB flush,
-// G = 2, 4, 8, D = 64 and 128): grids under 512 workgroups run 0.3-1.9 us
-// faster with 8 waves than with 4 (B=1 ctx 1024: 11.8 vs 13.7 us; ctx 16384:
-// 20.8 vs 21.4 us), and 16 waves are slower than 8 everywhere; from 512
-// workgroups up, 4 waves win.  The matrix-core kernel (two pages per round
-// trip) measured the same way picks the same: 4 waves at B = 8 x 8192 tokens
-// (8 waves -2%), 8 at B = 1 (equal or better).
-template <int G>
-static int gqa_waves(const DecodeArgs& a) {
-    const int64_t wgs = a.batch * a.hkv * a.num_splits;
-    return wgs * 4 >= kGqaManyWaves ? 4 : 8;
-}
-
 // Whether all `wgs` workgroups of a launch of KERNEL are resident at once,
 // the case in which the grouped-query kernels balance their waves by issue
 // priority (progress_priority).  Workgroups per CU come from the runtime's
@@ -1214,51 +1285,89 @@ static bool one_round(int threads, int64_t wgs) {
     return per_cu > 0 && wgs <= (int64_t)per_cu * cus;
 }
 
+// Balanced splits: the workgroups per kv head, or 0 where fixed splits serve.
+//   * One sequence has nothing to balance, and up to 1024 tokens the fixed
+//     splits leave each workgroup one or two iterations (8 x 700-1024 tokens,
+//     Hq=32, Hkv=8: 10.8 us fixed, 11.3 balanced; above, balanced is faster or
+//     equal: 2 x 4096 13.1 -> 12.6 us).
+//   * More than 64 sequences do not fit one load of lengths by a wave; a batch
+//     that large fills the GPU by itself.
+//   * Workgroups in whole rounds of the GPU: one 8-wave workgroup per CU
+//     (grouped-query kernels), two 4-wave ones (one head, D = 128), or as many
+//     rounds of those as give every sequence a workgroup and leave some to cut
+//     the longer ones: an eighth of the batch, half of it past 8192 tokens (one
+//     long sequence among short ones; the fixed rule splits there too), none
+//     for one head at D = 128, whose four waves of 16 loads gain less from a
+//     cut than a partial second round costs (16 x 100-1200 tokens, Hkv=32: 39.0
+//     us in 512 workgroups, 43.8 in up to 1024).  Where that leaves less than
+//     an eighth, the fixed splits' cheaper start wins (64 of 1-4096, Hkv=32:
+//     367.3 us against 368.3).
+// Measured against fixed splits of decode_partition (us a call, back to back;
+// Hq=32, Hkv=8, D=128 unless noted): 16 x 8192 88.9 -> 83.6; 16 ragged 512-8192
+// 65.4 -> 54.6, with Hq=64 77.6 -> 60.9; 32 ragged 64-4096 62.9 -> 55.4; 8 of
+// 500-32000, Hq=16 118.8 -> 103.5; 10 x 22420, D=64 82.9 -> 74.4; 8 x 32768,
+// Hkv=32 678 -> 652 (D=64: 366 -> 331).  768, 1024, 2048 and 4096 workgroups
+// where these rules take 256 or 512 were 1-30% slower.
+int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
+    if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24)) return 0;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    const bool one_head = hq == hkv && d == 128;
+    const int64_t round = one_head ? 2 * cus : cus;
+    const int64_t need = batch + (max_ctx > 8192 ? batch / 2 : one_head ? 0 : (batch + 7) / 8);
+    const int64_t workers = (need * hkv + round - 1) / round * round / hkv;
+    return workers * 8 < batch * 9 ? 0 : workers;  // next to no room to cut anything: fixed splits
+}
+
 template <int D, int G>
 static hipError_t launch_decode(const DecodeArgs& a) {
     int bs_shift = -1;
     for (int s = 0; s < 31; ++s)
         if ((int64_t(1) << s) == a.bs) bs_shift = s;
     const hipStream_t stream = (hipStream_t)a.stream;
-    dim3 grid((unsigned)a.hkv, (unsigned)a.num_splits, (unsigned)a.batch);
+    const dim3 grid((unsigned)a.hkv, (unsigned)a.num_splits, a.balanced ? 1u : (unsigned)a.batch);
     // Few enough splits: the last split of each (sequence, kv head) merges them
     // in the decode kernel (no reduce launch); otherwise the reduce kernel does.
-    int32_t* counters = a.counters && a.num_splits > 1 && a.num_splits <= kFusedMaxSplits ? a.counters : nullptr;
-    if constexpr (G == 1)
-        hipLaunchKernelGGL((paged_decode_kernel<D>), grid, dim3(DecodeTile<D>::THREADS), 0, stream, (const f16*)a.q,
-                           (const f16*)a.k_cache, (const f16*)a.v_cache, a.block_tables, a.context_lens,
-                           (f16*)a.out, a.o_part, a.m_part, a.l_part, counters, (int)a.hkv, (int)a.bs, bs_shift,
-                           (int)a.max_blocks, (int)a.num_blocks, (int)a.partition, (int)a.num_splits, a.sl2);
-    else {
-        const int64_t wgs = a.batch * a.hkv * a.num_splits;
-        auto launch = [&](auto nw) {
-            constexpr int NW = decltype(nw)::value, THREADS = GqaTile<D, G, NW>::THREADS;
-            const int balance = one_round<paged_decode_gqa_kernel<D, G, NW, gqa_pipelined(D, G)>>(THREADS, wgs);
-            hipLaunchKernelGGL((paged_decode_gqa_kernel<D, G, NW, gqa_pipelined(D, G)>), grid, dim3(THREADS), 0,
-                               stream, (const f16*)a.q, (const f16*)a.k_cache, (const f16*)a.v_cache,
-                               a.block_tables, a.context_lens, (f16*)a.out, a.o_part, a.m_part, a.l_part, counters,
-                               (int)a.hkv, (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks,
-                               (int)a.partition, (int)a.num_splits, a.sl2, balance);
+    int32_t* counters =
+        a.counters && a.num_splits > 1 && (a.balanced || a.num_splits <= kFusedMaxSplits) ? a.counters : nullptr;
+    auto launch = [&](auto* kernel, int threads, auto... more) {
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, (const f16*)a.q, (const f16*)a.k_cache,
+                           (const f16*)a.v_cache, a.block_tables, a.context_lens, (f16*)a.out, a.o_part, a.m_part,
+                           a.l_part, counters, (int)a.hkv, (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks,
+                           (int)a.partition, (int)a.num_splits, a.sl2, more..., (int)a.balanced, (int)a.batch,
+                           (int)a.token_cap);
+    };
+    if constexpr (G == 1) {
+        launch(paged_decode_kernel<D>, DecodeTile<D>::THREADS);
+    } else {
+        const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+        auto launch_nw = [&](auto nw) {
+            constexpr int NW = decltype(nw)::value;
+            if constexpr (G == 8) {
+                constexpr auto K = paged_decode_gqa_mfma_kernel<D, G, NW>;
+                launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
+            } else {
+                constexpr auto K = paged_decode_gqa_kernel<D, G, NW, gqa_pipelined(D, G)>;
+                launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
+            }
         };
-        auto launch_mfma = [&](auto nw) {
-            constexpr int NW = decltype(nw)::value, THREADS = GqaMfmaTile<D, G, NW>::THREADS;
-            const int balance = one_round<paged_decode_gqa_mfma_kernel<D, G, NW>>(THREADS, wgs);
-            hipLaunchKernelGGL((paged_decode_gqa_mfma_kernel<D, G, NW>), grid, dim3(THREADS), 0, stream,
-                               (const f16*)a.q, (const f16*)a.k_cache, (const f16*)a.v_cache, a.block_tables,
-                               a.context_lens, (f16*)a.out, a.o_part, a.m_part, a.l_part, counters, (int)a.hkv,
-                               (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks, (int)a.partition,
-                               (int)a.num_splits, a.sl2, balance);
-        };
-        const bool many = gqa_waves<G>(a) == 4;
-        if constexpr (G == 8) {
-            if (many)
-                launch_mfma(std::integral_constant<int, 4>{});
-            else
-                launch_mfma(std::integral_constant<int, 8>{});
-        } else if (many)
-            launch(std::integral_constant<int, 4>{});
+        // Waves per workgroup of both grouped-query kernels.  A dot-product wave
+        // reads one 16-token page per round trip to memory, so a split of P tokens
+        // costs P / (16 NW) dependent round trips; with many workgroups per CU they
+        // overlap, but in a small grid (one sequence, few kv heads) they are the
+        // kernel's critical path.  Measured on MI355X (one call after a 512 MiB flush,
+        // G = 2, 4, 8, D = 64 and 128): grids under 512 workgroups run 0.3-1.9 us
+        // faster with 8 waves than with 4 (B=1 ctx 1024: 11.8 vs 13.7 us; ctx 16384:
+        // 20.8 vs 21.4 us), and 16 waves are slower than 8 everywhere; from 512
+        // workgroups up, 4 waves win.  The matrix-core kernel (two pages per round
+        // trip) measured the same way picks the same: 4 waves at B = 8 x 8192 tokens
+        // (8 waves -2%), 8 at B = 1 (equal or better).
+        if (wgs * 4 >= kGqaManyWaves)
+            launch_nw(std::integral_constant<int, 4>{});
         else
-            launch(std::integral_constant<int, 8>{});
+            launch_nw(std::integral_constant<int, 8>{});
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.num_splits == 1 || counters) return e;

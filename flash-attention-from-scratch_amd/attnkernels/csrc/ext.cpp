@@ -121,8 +121,10 @@ torch::Tensor flash_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor v, to
     return o;
 }
 
-torch::Tensor paged_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor bt,
-                           torch::Tensor ctx, int64_t max_ctx, double scale, int64_t partition) {
+// balanced: splits cut by the kernel from the context lengths, where they serve.
+static torch::Tensor decode(const torch::Tensor& q, const torch::Tensor& kc, const torch::Tensor& vc,
+                            const torch::Tensor& bt, const torch::Tensor& ctx, int64_t max_ctx, double scale,
+                            int64_t partition, bool balanced) {
     TORCH_CHECK(q.is_cuda() && q.scalar_type() == torch::kHalf && q.dim() == 3 && q.is_contiguous(),
                 "q must be a contiguous fp16 GPU tensor [B, H, D]");
     TORCH_CHECK(kc.is_cuda() && kc.scalar_type() == torch::kHalf && kc.dim() == 4 && kc.is_contiguous() &&
@@ -138,18 +140,30 @@ torch::Tensor paged_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, 
     const at::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
     auto out = torch::empty_like(q);
     const int64_t B = q.size(0), hq = q.size(1), D = q.size(2), hkv = kc.size(1);
-    const size_t ws_bytes = ak_paged_decode_workspace_size(B, hq, D, max_ctx, partition);
+    size_t ws_bytes = balanced ? ak_paged_decode_balanced_workspace_size(B, hq, hkv, D, max_ctx, partition) : 0;
+    const auto run = ws_bytes > 0 ? ak_paged_decode_balanced : ak_paged_decode_fused;
+    if (ws_bytes == 0) ws_bytes = ak_paged_decode_workspace_size(B, hq, D, max_ctx, partition);
     torch::Tensor ws, counters;
     if (ws_bytes > 0) {
         ws = torch::empty({(int64_t)ws_bytes}, q.options().dtype(torch::kByte));
         counters = split_counters(q, B * hkv);
     }
-    check_rc(ak_paged_decode_fused(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), bt.data_ptr<int32_t>(),
-                                   ctx.data_ptr<int32_t>(), out.data_ptr(), B, hq, hkv, D, kc.size(0), kc.size(2),
-                                   bt.size(1), max_ctx, scale, partition, ws_bytes ? ws.data_ptr() : nullptr,
-                                   ws_bytes, ws_bytes ? counters.data_ptr<int32_t>() : nullptr,
-                                   ws_bytes ? counters.numel() : 0, stream_of(q)));
+    check_rc(run(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), bt.data_ptr<int32_t>(), ctx.data_ptr<int32_t>(),
+                 out.data_ptr(), B, hq, hkv, D, kc.size(0), kc.size(2), bt.size(1), max_ctx, scale, partition,
+                 ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, ws_bytes ? counters.data_ptr<int32_t>() : nullptr,
+                 ws_bytes ? counters.numel() : 0, stream_of(q)));
     return out;
+}
+
+torch::Tensor paged_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor bt,
+                           torch::Tensor ctx, int64_t max_ctx, double scale, int64_t partition) {
+    return decode(q, kc, vc, bt, ctx, max_ctx, scale, partition, false);
+}
+
+// Splits of about equal size where they serve, else of `partition` tokens.
+torch::Tensor paged_decode_balanced(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor bt,
+                                    torch::Tensor ctx, int64_t max_ctx, double scale, int64_t partition) {
+    return decode(q, kc, vc, bt, ctx, max_ctx, scale, partition, true);
 }
 
 // In place: writes key/value rows into the caches (no counterpart in the
@@ -208,6 +222,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("flash_simt", &flash_simt, "prefill attention (served by the MFMA flash kernel)");
     m.def("flash_wmma", &flash_wmma, "tiled attention with online softmax on MFMA matrix cores");
     m.def("paged_decode", &paged_decode, "decode attention over a paged KV cache, split-K");
+    m.def("paged_decode_balanced", &paged_decode_balanced, "the same with splits cut evenly over the batch's contexts");
     m.def("stream_checksum", &stream_checksum, "XOR checksum of a tensor's bytes (read-only streaming ceiling)",
           py::arg("x"), py::arg("out") = py::none());
     m.def("reshape_and_cache", &reshape_and_cache, "write new tokens' K/V rows into the paged caches");

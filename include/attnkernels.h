@@ -137,6 +137,26 @@ int ak_paged_decode_fused(const void *q, const void *k_cache, const void *v_cach
                           int64_t max_context_len, double scale, int64_t partition, void *workspace,
                           size_t workspace_bytes, int32_t *counters, int64_t counters_len, void *stream);
 
+/* Paged-KV decode whose splits the kernel cuts itself, of about equal size,
+ * from the context lengths it finds on the device: a ragged batch then keeps
+ * every compute unit busy to the end, which splits of one fixed size do not.
+ * No counterpart in the reference (its splits are `partition` tokens each,
+ * attnkernels/csrc/paged_decode.cu:73-77).  The size function returns the bytes
+ * of the workspace on the current device, or 0 for sizes that fixed splits
+ * serve (one sequence, more than 64, max_context_len up to 1024, invalid
+ * sizes): the call is then refused with AK_ERR_UNSUPPORTED.  `partition` only
+ * bounds the tokens read of a sequence, as in ak_paged_decode: those below the
+ * smallest multiple of it >= max_context_len.  counters is required.  Arguments,
+ * results and errors are otherwise those of ak_paged_decode_fused. */
+size_t ak_paged_decode_balanced_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                               int64_t head_dim, int64_t max_context_len, int64_t partition);
+int ak_paged_decode_balanced(const void *q, const void *k_cache, const void *v_cache,
+                             const int32_t *block_tables, const int32_t *context_lens, void *out,
+                             int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                             int64_t num_blocks, int64_t block_size, int64_t max_blocks_per_seq,
+                             int64_t max_context_len, double scale, int64_t partition, void *workspace,
+                             size_t workspace_bytes, int32_t *counters, int64_t counters_len, void *stream);
+
 /* Paged-KV decode that allocates nothing: ak_paged_decode without the
  * workspace arguments.  No counterpart in the reference; it is for callers
  * that cannot allocate device memory (code under HIP graph capture, tight

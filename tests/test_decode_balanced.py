@@ -1,0 +1,52 @@
+"""Decode with splits cut evenly over the batch (no partition given): every
+kernel, at the edges of the cut, against the oracle; the counters are back at
+zero after each call (the next one, with other lengths, would merge too early)."""
+import numpy as np
+import pytest
+import torch
+
+import attnkernels as ak
+import oracle
+from conftest import TOL, max_err
+
+pytestmark = pytest.mark.gpu
+
+BATCHES = {
+    "edges": [1, 255, 256, 257, 1279, 1280, 1281, 2048],
+    "skewed": [20000] + [3] * 15,
+    "full": [1100 + 7 * i for i in range(64)],       # the most sequences, a lane each
+    "two": [1, 4099],
+    "empty": [0, 1500, 0, 2049, 0],                  # outside the >= 1 contract: zero rows
+}
+
+
+@pytest.mark.parametrize("name", BATCHES)
+@pytest.mark.parametrize("g,hkv,d,bs", [(1, 4, 128, 16), (1, 2, 64, 8), (2, 2, 128, 16), (4, 8, 128, 16),
+                                        (4, 2, 64, 32), (8, 4, 128, 16), (8, 2, 64, 12)])
+def test_matches_oracle(name, g, hkv, d, bs):
+    lens = BATCHES[name]
+    kc, vc, bt, cl = oracle.make_paged_cache([max(1, n) for n in lens], hkv, d, block_size=bs, extra_blocks=3, seed=g)
+    cl[:] = lens
+    q = np.random.default_rng(g + d).standard_normal((len(lens), g * hkv, d), dtype=np.float32).astype(np.float16)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, bt, cl)]
+    rows = [b for b, n in enumerate(lens) if n > 0]
+    ref = np.zeros(q.shape, np.float32)
+    ref[rows] = oracle.paged_decode_fp32(q[rows], kc, vc, bt[rows], cl[rows])
+    for _ in range(2):
+        assert max_err(ak.paged_decode(*dev, max(lens)), ref) < TOL[d]
+    # other lengths right after, on the same counters
+    dev[4] = torch.clamp(dev[4] // 2, min=1)
+    short = cl // 2
+    short[short < 1] = 1
+    assert max_err(ak.paged_decode(*dev, max(lens)), oracle.paged_decode_fp32(q, kc, vc, bt, short)) < TOL[d]
+
+
+def test_tokens_past_the_longest_context_given_are_cut_as_with_fixed_splits():
+    """A length above max_context_len (outside the contract) reads up to the end of the last fixed split."""
+    kc, vc, bt, cl = oracle.make_paged_cache([6000, 300], 2, 128, block_size=16, extra_blocks=1, seed=1)
+    q = np.random.default_rng(2).standard_normal((2, 8, 128), dtype=np.float32).astype(np.float16)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, bt, cl)]
+    part = ak.decode_partition(2, 2, 3000)
+    a = ak.paged_decode(*dev, 3000)
+    b = ak.paged_decode(*dev, 3000, partition_size=part)
+    assert max_err(a, b.float().cpu().numpy()) < 1e-3

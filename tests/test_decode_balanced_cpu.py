@@ -1,0 +1,140 @@
+"""The cut of a batch's contexts into splits that the decode kernels make when
+no partition is given (balanced_segment in decode.hip), replayed lane by lane in
+float32 and int32, and the rule that picks that path (decode_balanced_workers).
+
+Every split must hold a token, the splits of a sequence must tile its context,
+and no kv head may need more splits than the launch has workgroups: a split
+that is never run, or that holds nothing and so never arrives at the merge,
+would leave its sequence without an output."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import PKG_DIR
+
+F = np.float32
+MIN_SPLIT, MAX_BATCH = 256, 64
+
+
+def rcp(x, ulp):
+    """1 / x as a hardware reciprocal may return it: off by one unit in the last place."""
+    r = F(1) / F(x)
+    return np.nextafter(r, F(np.inf if ulp > 0 else -np.inf)) if ulp else r
+
+
+def cut(lens, workers, cap, gran, ulp=0):
+    c = np.minimum(np.maximum(np.asarray(lens, np.int64), 0), cap)
+
+    def up(x):
+        return (int(x) + gran - 1) // gran * gran
+
+    size = max(MIN_SPLIT, up(1 + int(F(c.sum() - 1) * rcp(workers, ulp))))
+    for it in range(9):
+        n = (c.astype(F) * rcp(size, ulp)).astype(np.int64)
+        n += n * size < c
+        n -= (n - 1) * size >= c
+        n = np.maximum(1, n)
+        count = int(n.sum())
+        if count <= workers:
+            break
+        size = up(size + 1 + int(F(size) * F(count - workers) * rcp(workers, ulp))) if it < 6 else up(cap)
+    segs = []
+    for b, (ctx, ns) in enumerate(zip(c, n)):
+        length = up((ctx + ns - 1) // ns)
+        segs += [(b, s, int(ns), s * length, min(int(ctx), (s + 1) * length)) for s in range(ns)]
+    return segs, count, size
+
+
+def batches():
+    rng = np.random.default_rng(0)
+    yield [0, 1, 256, 257, 1025]
+    yield [1025] * MAX_BATCH
+    yield [32768] + [1] * 31
+    yield [0] * 7 + [5000]
+    yield [(1 << 24) - 257, 1]
+    for _ in range(400):
+        batch, high = int(rng.integers(2, MAX_BATCH + 1)), int(2 ** rng.uniform(10, 17))
+        yield rng.integers(0 if rng.random() < 0.3 else 1, high + 1, batch).tolist()
+
+
+@pytest.mark.parametrize("gran", [64, 128, 256])  # tokens of a workgroup's iteration, over all kernels
+@pytest.mark.parametrize("ulp", [-1, 0, 1])
+def test_every_token_is_in_one_split(gran, ulp):
+    for lens in batches():
+        cap = -(-max(lens) // 256) * 256
+        for workers in (len(lens), len(lens) + 1, 2 * len(lens), 300):
+            segs, count, size = cut(lens, workers, cap, gran, ulp)
+            assert count <= workers and size % gran == 0, (lens, workers)
+            at = {}
+            for b, s, ns, start, end in segs:
+                assert start == at.get(b, 0) and (end > start or lens[b] == 0), (lens, workers, b, s)
+                at[b] = end
+            assert [at[b] for b in range(len(lens))] == lens, (lens, workers)
+
+
+def test_even_batches_are_cut_evenly():
+    for batch, workers, ctx in ((16, 32, 8192), (8, 32, 8192), (4, 64, 30000), (10, 32, 22420)):
+        segs, _, _ = cut([ctx] * batch, workers, ctx + 255, 128)
+        assert len(segs) == workers // batch * batch
+        assert max(e - s for _, _, _, s, e in segs) <= ctx // (workers // batch) + 128
+
+
+def test_a_cut_that_rounds_up_its_count_is_caught():
+    """With a float ceiling alone (no step of correction) 2 * size tokens can count as 3 splits, one of them empty."""
+    size, ctx = 128, 256
+    n = int(np.ceil(F(ctx) * rcp(size, 1)))
+    length = -(-(-(-ctx // n)) // 128) * 128
+    assert n == 3 and (n - 1) * length >= ctx
+
+
+@pytest.fixture(scope="module")
+def lib():
+    L = ctypes.CDLL(str(PKG_DIR / "attnkernels" / "libattnkernels.so"))
+    vp, i64, f64 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_double
+    L.ak_last_error.restype = ctypes.c_char_p
+    L.ak_paged_decode_balanced_workspace_size.argtypes = [i64] * 6
+    L.ak_paged_decode_balanced_workspace_size.restype = ctypes.c_size_t
+    L.ak_paged_decode_balanced.argtypes = [vp] * 6 + [i64] * 8 + [f64, i64, vp, ctypes.c_size_t, vp, i64, vp]
+    return L
+
+
+def workers(lib, batch, hq, hkv, d, max_ctx, partition=1024):
+    size = lib.ak_paged_decode_balanced_workspace_size(batch, hq, hkv, d, max_ctx, partition)
+    assert size % (hq * (d + 2) * 4) == 0
+    return size // (hq * (d + 2) * 4)
+
+
+def test_rule(lib):
+    # fixed splits: one sequence, more than 64, short contexts, lengths past 2^24, invalid sizes
+    for args in ((1, 32, 8, 128, 8192), (65, 32, 8, 128, 8192), (16, 32, 8, 128, 1024), (16, 32, 8, 128, 1 << 24),
+                 (16, 32, 0, 128, 8192), (16, 30, 8, 128, 8192), (0, 32, 8, 128, 8192)):
+        assert workers(lib, *args) == 0, args
+    assert workers(lib, 16, 32, 8, 128, 8192, 0) == 0
+    # every sequence has a workgroup, and whole rounds of 256 CUs (512 slots for one head at D = 128) of them
+    for batch in (2, 3, 16, 33, 64):
+        for hq, hkv in ((32, 32), (32, 8), (64, 8), (4, 4), (40, 5), (600, 600)):
+            for d in (64, 128):
+                for ctx in (1025, 8192, 8193, 100000):
+                    w = workers(lib, batch, hq, hkv, d, ctx)
+                    if w == 0:  # no room to cut: about one workgroup per sequence
+                        assert hq == hkv and d == 128 and ctx <= 8192
+                        continue
+                    assert w >= batch + (batch // 2 if ctx > 8192 else 0) and w <= 65535
+                    unit = 512 if hq == hkv and d == 128 else 256
+                    assert w * hkv % unit > unit - hkv or w * hkv % unit == 0
+    assert workers(lib, 16, 32, 8, 128, 8192) == 32 and workers(lib, 16, 32, 32, 128, 8192) == 0 and workers(lib, 8, 32, 32, 128, 8192) == 16
+
+
+def test_refused_calls(lib):
+    fake = ctypes.c_void_p(4096)
+
+    def call(batch=4, hq=32, hkv=8, max_ctx=4096, partition=1024, ws=fake, ws_bytes=1 << 30, counters=fake, n=1 << 20):
+        return lib.ak_paged_decode_balanced(fake, fake, fake, fake, fake, fake, batch, hq, hkv, 128, 10, 16, 512,
+                                            max_ctx, 0.1, partition, ws, ws_bytes, counters, n, None)
+
+    assert call(batch=1) == 2 and b"fixed splits" in lib.ak_last_error()
+    assert call(partition=100) == 1 and lib.ak_last_error() == b"partition size must be a positive multiple of 256"
+    assert call(hq=30) == 1 and call(max_ctx=0) == 1
+    assert call(counters=None) == 1 and call(n=31) == 1 and b"counters" in lib.ak_last_error()
+    assert call(ws=None) == 3 and call(ws_bytes=100) == 3 and call(ws=ctypes.c_void_p(4100)) == 1
