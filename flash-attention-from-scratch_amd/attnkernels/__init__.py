@@ -198,7 +198,8 @@ def paged_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_le
     partition_size: tokens per split (multiple of 256); a value >= max_context_len
                   disables split-K.  None: the kernel cuts the contexts into splits
                   of about equal size; where it does not (one sequence, more than
-                  64, contexts up to 1024 tokens), decode_partition picks one.
+                  64, contexts up to 1024 tokens, less than 64 MB of K and V
+                  at max_context_len), decode_partition picks one.
     """
     if not (q.dtype == k_cache.dtype == v_cache.dtype == torch.float16):
         raise ValueError("q and caches must be fp16")

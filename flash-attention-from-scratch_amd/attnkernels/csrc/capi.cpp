@@ -65,7 +65,7 @@ int prefill(const char* who, const void* q, const void* k, const void* v, void* 
     a.hkv = kv_heads;
     a.cu = cu;
     a.total_rows = total_rows;
-    a.n = seq_len;
+    a.n = cu ? std::min(seq_len, total_rows) : seq_len;  // packed: no sequence has more rows than there are
     a.d = (int)head_dim;
     a.causal = causal != 0;
     // |scale| * log2(e), kept >= 1e-30 so that masked scores (-inf) still map to

@@ -1286,10 +1286,12 @@ static bool one_round(int threads, int64_t wgs) {
 }
 
 // Balanced splits: the workgroups per kv head, or 0 where fixed splits serve.
-//   * One sequence has nothing to balance, and up to 1024 tokens the fixed
-//     splits leave each workgroup one or two iterations (8 x 700-1024 tokens,
-//     Hq=32, Hkv=8: 10.8 us fixed, 11.3 balanced; above, balanced is faster or
-//     equal: 2 x 4096 13.1 -> 12.6 us).
+//   * One sequence has nothing to balance; up to 1024 tokens, or 64 MB of K and
+//     V if all were the longest, the fixed splits leave each workgroup a few
+//     iterations, and finding the cut costs up to 0.5 us more than it gives (8 x
+//     700-1024 tokens, Hq=32, Hkv=8: 10.8 us fixed, 11.3 balanced; 3 x 8100,
+//     Hq=16, Hkv=4: 14.3 fixed, 14.9 balanced; 4 x 300-9000, 8 heads, 147 MB:
+//     31.1 fixed, 23.3 balanced).
 //   * More than 64 sequences do not fit one load of lengths by a wave; a batch
 //     that large fills the GPU by itself.
 //   * Workgroups in whole rounds of the GPU: one 8-wave workgroup per CU
@@ -1309,7 +1311,9 @@ static bool one_round(int threads, int64_t wgs) {
 // Hkv=32 678 -> 652 (D=64: 366 -> 331).  768, 1024, 2048 and 4096 workgroups
 // where these rules take 256 or 512 were 1-30% slower.
 int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
-    if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24)) return 0;
+    if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24) ||
+        batch * hkv * max_ctx * d * 4 < (int64_t(64) << 20))
+        return 0;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)

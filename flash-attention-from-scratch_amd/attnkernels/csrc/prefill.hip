@@ -10,17 +10,18 @@
 //     each wave owns 32 of them, so no softmax row is shared between waves.
 //     Eight waves share each K/V tile in LDS: half the LDS traffic per query
 //     row of a 4-wave workgroup, and each wave issues only 2 one-KB loads per
-//     K and per V tile.  Short sequences and small grids use 4-wave workgroups
-//     (128 rows, two per CU; at D = 64 with 64-key tiles, three per CU)
-//     instead: see prefill_waves.
-//   * Two MFMA shapes, chosen per launch (prefill_mfma16): M = 32
+//     K and per V tile.  Short sequences and mid-size grids use 4-wave
+//     workgroups (128 rows, two per CU; at D = 64 with 64-key tiles, three per
+//     CU) instead, and small grids teams of waves that share their query rows
+//     and split the key tiles: see prefill_plan.
+//   * Two MFMA shapes, chosen per launch (prefill_plan): M = 32
 //     (v_mfma_f32_32x32x16_f16) and M = 16 (v_mfma_f32_16x16x32_f16).  On
 //     MI355X the 16x16 form costs less energy per FLOP: a matrix-core-only loop
 //     at two waves per SIMD sustains 1.9-2.0 PFLOP/s on random fp16 data
 //     against 1.2-1.6 for 32x32, and the D = 128 kernel runs at a 12% higher
 //     clock with it.  It also issues twice the MFMA instructions, so it pays
 //     only where the key loop is long: D = 128 with 8-wave workgroups, causal
-//     N >= 6144 and non-causal N >= 3072.
+//     (single tiles) and non-causal N >= 3072, causal pairs N >= 6144.
 //   * Scores are computed transposed, S^T = K Q^T, with K as the MFMA A operand
 //     (16-byte LDS reads of K rows) and Q as the B operand (kept in VGPRs for
 //     the whole kernel).
@@ -56,14 +57,21 @@
 //     t into P (exponentials, fp16 conversion, row sums), then P V of tile t
 //     follows.  sched_group_barrier fixes that interleave.  K is therefore
 //     loaded two tiles ahead and V one tile ahead.
-//   * Causal: a workgroup processes query tile j and tile nqt-1-j, so every
-//     workgroup has the same amount of work; waves skip key tiles that lie
+//   * Causal: a workgroup processes one query tile, the heaviest tiles of all
+//     slices first, or (long sequences on large grids) tile j and tile nqt-1-j,
+//     so that all have the same amount of work; waves skip key tiles that lie
 //     entirely above their diagonal; masking runs only on diagonal/tail tiles.
+//   * Teams (KG > 1): KG groups of NW waves work on the same query rows, team k
+//     on key tiles k, k + KG, ..., each with its own ring of tiles; at the end
+//     their O, m and l are merged through LDS.  This shortens the chain of key
+//     tiles that bounds a grid of no more workgroups than CUs.
 //   * Workgroup ids are remapped so that the query tiles of one (batch, head)
 //     run on the same XCD and share its L2.
 #include "attn_kernels.hpp"
 #include "wave.hpp"
 
+#include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #define AK_LDS __attribute__((address_space(3)))
@@ -76,7 +84,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 template <int D, int NWAVES, int M>
 struct PrefillTile {
     static_assert(M == 16 || M == 32, "MFMA shape");
-    static constexpr int NW = NWAVES;            // waves per workgroup: 8, or 4 for short sequences
+    static constexpr int NW = NWAVES;            // waves per query tile (of each team)
     static constexpr int THREADS = NW * kWave;   // 512 or 256
     static constexpr int QW = 32;                // query rows per wave
     static constexpr int QB = 32 / M;            // query blocks per wave (one per row a lane owns)
@@ -85,8 +93,9 @@ struct PrefillTile {
     // Keys per tile: a K tile is 16 KB (64 keys at D = 128, 128 at D = 64), except
     // for D = 64 in 4-wave workgroups, whose 64-key tiles keep the wave under
     // 168 VGPRs, so that a CU holds three of those workgroups (+5-9% on short
-    // sequences; with 8 waves the 128-key tile is 2-4% faster).
-    static constexpr int BN = D == 64 && NW == 4 ? 64 : 8192 / D;
+    // sequences; with 8 waves the 128-key tile is 2-4% faster), and the teams of
+    // one or two waves, four of which fit the LDS of a CU with 8 KB tiles.
+    static constexpr int BN = NW <= 2 ? 4096 / D : D == 64 && NW == 4 ? 64 : 8192 / D;
     static constexpr int TILE = BN * D;          // halves per K (or V) tile
     static constexpr int STAGE = 2 * TILE;       // K + V
     static constexpr int RPI = 512 / D;          // rows per 1 KB load instruction
@@ -513,12 +522,13 @@ struct PrefillSched {
     static constexpr int MF_EXP = M == 16 ? (E2 ? ceil_div(E2, NPV) : 0) : 2;
 };
 
-// Software-pipelined key loop: iteration t multiplies the scores of tile t
+// Software-pipelined key loop (KG teams: of team kg's tiles, keys
+// (t KG + kg) BN on): iteration t multiplies the scores of tile t
 // (computed one iteration earlier) into O while the matrix core computes the
 // scores of tile t+1, so the exponentials of one tile overlap the QK^T MFMAs
 // of the next inside every wave.  K runs two tiles ahead in a 2-buffer ring,
 // V one tile ahead in another; one barrier per tile.
-template <int D, bool CAUSAL, int NW, int M>
+template <int D, bool CAUSAL, int NW, int M, int KG>
 __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, const f16* __restrict__ kb,
                                               const f16* __restrict__ vb, f16* __restrict__ ob,
                                               f16* __restrict__ lds, int q0, int n, int qs, int ks, float sl2,
@@ -526,20 +536,22 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
     using T = PrefillTile<D, NW, M>;
     using SC = PrefillSched<D, NW, M>;
     const int tid = threadIdx.x;
-    const int lane = tid & 63, w = uniform(tid >> 6);
+    const int lane = tid & 63, wave = uniform(tid >> 6);
+    const int w = KG == 1 ? wave : wave % NW, kg = KG == 1 ? 0 : wave / NW;
     const int qw0 = q0 + w * T::QW;
-    f16* kbuf = lds;                 // 2 K tiles
-    f16* vbuf = lds + 2 * T::TILE;   // 2 V tiles
+    f16* kbuf = lds + kg * 2 * T::STAGE;  // 2 K tiles
+    f16* vbuf = kbuf + 2 * T::TILE;       // 2 V tiles
 
     const int kend = CAUSAL ? min(n, q0 + T::BM) : n;
-    const int nkt = (kend + T::BN - 1) / T::BN;
+    const int nkt = (kend + T::BN * KG - 1) / (T::BN * KG);
     // Tiles before kt_mask need no masking for any wave of the workgroup: all
     // their keys are < n and (causal) <= the workgroup's first query row.
-    const int kt_mask = min(nkt, CAUSAL ? q0 / T::BN : n / T::BN);
+    const int kt_mask = min(nkt, (CAUSAL ? q0 : n) / (T::BN * KG));
+    auto key0 = [&](int t) { return (t * KG + kg) * T::BN; };  // first key of this team's tile t
 
-    load_kv<D, false, NW, M>(kb, kbuf, 0, n, ks, w, lane);
-    load_kv<D, true, NW, M>(vb, vbuf, 0, n, ks, w, lane);
-    if (nkt > 1) load_kv<D, false, NW, M>(kb, kbuf + T::TILE, T::BN, n, ks, w, lane);
+    load_kv<D, false, NW, M>(kb, kbuf, key0(0), n, ks, w, lane);
+    load_kv<D, true, NW, M>(vb, vbuf, key0(0), n, ks, w, lane);
+    if (nkt > 1) load_kv<D, false, NW, M>(kb, kbuf + T::TILE, key0(1), n, ks, w, lane);
 
     // Q as the MFMA B operand: col = query, k = KK head dims per step.
     QFrag<D, NW, M> qf;
@@ -578,7 +590,7 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
         constexpr bool MASK = decltype(mask_tag)::value;
         constexpr bool LAST = decltype(last_tag)::value;  // the last tile: no next S to compute
         wait_loads_and_sync();  // K(t+1), V(t) landed; nobody reads K(t), V(t-1) any more
-        if (t + 2 < nkt) load_kv<D, false, NW, M>(kb, kbuf + (t & 1) * T::TILE, (t + 2) * T::BN, n, ks, w, lane);
+        if (t + 2 < nkt) load_kv<D, false, NW, M>(kb, kbuf + (t & 1) * T::TILE, key0(t + 2), n, ks, w, lane);
         // V(t+1) goes to the slot of V(t-1), last read before this barrier.  D = 64
         // issues it here; D = 128 after its QK^T phase, which spreads the CU's tile
         // loads over the tile (+1-2% at D = 128, -8-10% at D = 64).  Every body but
@@ -587,16 +599,17 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
         // unrolled body's exponentials out of the QK^T interleave, below the branch.
         constexpr bool V_LATE = D == 128;
         if (!V_LATE && !LAST)
-            load_kv<D, true, NW, M>(vb, vbuf + ((t + 1) & 1) * T::TILE, (t + 1) * T::BN, n, ks, w, lane);
+            load_kv<D, true, NW, M>(vb, vbuf + ((t + 1) & 1) * T::TILE, key0(t + 1), n, ks, w, lane);
         // Causal: a tile whose first key is after this wave's last row is skipped.
-        const bool act = !MASK || !CAUSAL || t * T::BN <= qw0 + T::QW - 1;
+        // So is one past the last key, which only a team of several meets.
+        const bool act = !MASK || ((!CAUSAL || key0(t) <= qw0 + T::QW - 1) && (KG == 1 || key0(t) < n));
         // The diagonal tiles of causal D = 64 take the tile's row maximum first; all
         // other tiles check the exponents after the fact (settle_part).
         // The split check on the masked tiles as well costs the causal D = 64 kernels
         // their register budget (spills at 8 waves, a third workgroup per CU at 4).
         constexpr bool MAX_FIRST = D == 64 && CAUSAL && MASK;
         if (act) {
-            if constexpr (MASK) mask_tile<D, NW, M, CAUSAL>(sc, t * T::BN, n, qw0, lane);
+            if constexpr (MASK) mask_tile<D, NW, M, CAUSAL>(sc, key0(t), n, qw0, lane);
             if constexpr (MAX_FIRST) max_tile<D, NW, M>(sc, o, st, sl2);
         }
         // The wave holds priority 1 while its QK^T MFMAs and exponentials run and
@@ -637,7 +650,7 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
         }
         __builtin_amdgcn_s_setprio(0);
         if (V_LATE && !LAST)
-            load_kv<D, true, NW, M>(vb, vbuf + ((t + 1) & 1) * T::TILE, (t + 1) * T::BN, n, ks, w, lane);
+            load_kv<D, true, NW, M>(vb, vbuf + ((t + 1) & 1) * T::TILE, key0(t + 1), n, ks, w, lane);
         if (act) {
             const f16* vt = vbuf + (t & 1) * T::TILE;
             if constexpr (MAX_FIRST) {
@@ -746,6 +759,54 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
     if (t < kt_mask) body(t, sx, sy, std::false_type{}, std::true_type{});
     else body(t, sx, sy, std::true_type{}, std::true_type{});
 
+    if constexpr (KG > 1) {
+        // The teams' O, m and l, merged by the LSE rule: the others leave theirs
+        // in LDS (16-byte pieces, a lane's pieces kWave apart), the first adds
+        // them to its own.
+        constexpr int R = M == 32 ? 16 : 4, PIECES = T::DT * T::QB * R / 4, WAVE = (PIECES * 4 + 2 * T::QB) * kWave;
+        static_assert((KG - 1) * NW * WAVE * 4 <= KG * 2 * T::STAGE * 2, "the merge fits the tiles' LDS");
+        float* const part = reinterpret_cast<float*>(lds) + w * WAVE;
+        __syncthreads();  // every wave is done with its tiles
+        if (kg > 0) {
+            float* dst = part + (kg - 1) * NW * WAVE;
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                f32x4 x;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = o[i * 4 / R / T::QB][i * 4 / R % T::QB][i * 4 % R + j];
+                *reinterpret_cast<f32x4*>(dst + (i * kWave + lane) * 4) = x;
+            }
+#pragma unroll
+            for (int qb = 0; qb < T::QB; ++qb) {
+                dst[PIECES * 4 * kWave + (2 * qb) * kWave + lane] = st.m[qb];
+                dst[PIECES * 4 * kWave + (2 * qb + 1) * kWave + lane] = st.l[qb];
+            }
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int k = 0; k < KG - 1; ++k) {
+            const float* src = part + k * NW * WAVE;
+            float wo[T::QB];
+#pragma unroll
+            for (int qb = 0; qb < T::QB; ++qb) {
+                const float mk = src[PIECES * 4 * kWave + (2 * qb) * kWave + lane];
+                // The first team holds key 0, so its m is finite; one without keys has m = -inf and weighs 0.
+                const float mx = fmaxf(st.m[qb], mk);
+                if (mx > st.m[qb]) move_max<D, NW, M>(st, o, qb, mx);
+                wo[qb] = exp2_fast(mk - mx);
+                st.l[qb] += wo[qb] * src[PIECES * 4 * kWave + (2 * qb + 1) * kWave + lane];
+            }
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                const f32x4 x = *reinterpret_cast<const f32x4*>(src + (i * kWave + lane) * 4);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    o[i * 4 / R / T::QB][i * 4 / R % T::QB][i * 4 % R + j] += wo[i * 4 / R % T::QB] * x[j];
+            }
+        }
+    }
+
     // O = O^T / l.
     //   M = 32: lane holds query l%32, head dims 32t + 16hh + 8(l/32) + i.
     //   M = 16: lane holds queries 16qb + l%16, head dims 16t + 4(l/16) + i.
@@ -785,21 +846,33 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
 // Packed layout (VARLEN): q/o [total, Hq, D], k/v [total, Hkv, D], sequence b
 // being rows cu[b] .. cu[b+1]-1; the grid is sized for the longest sequence and
 // the units past a shorter one exit before touching memory.
-template <int D, bool CAUSAL, bool VARLEN, int NW, int M>
-__global__ void __launch_bounds__((PrefillTile<D, NW, M>::THREADS)) __attribute__((amdgpu_waves_per_eu(2)))
+template <int D, bool CAUSAL, bool VARLEN, int NW, int M, int KG, bool SINGLE>
+__global__ void __launch_bounds__((PrefillTile<D, NW, M>::THREADS * KG)) __attribute__((amdgpu_waves_per_eu(2)))
 flash_prefill_kernel(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __restrict__ V,
                      f16* __restrict__ O, const int32_t* __restrict__ cu, int total_rows, int n_max,
-                     int units_per_bh, int total_units, int hq, int group, float sl2, uint32_t qflip) {
+                     int units_per_bh, int total_units, int span, int hq, int group, float sl2, uint32_t qflip) {
     using T = PrefillTile<D, NW, M>;
-    __shared__ __attribute__((aligned(1024))) f16 lds[2 * T::STAGE];
+    __shared__ __attribute__((aligned(1024))) f16 lds[KG * 2 * T::STAGE];
     // Dense: every (b, h) has the same units, so contiguous ranges per XCD are
     // balanced.  Varlen: the units past a short sequence are empty, so whole
     // GQA groups (all units of the query heads sharing a kv head) are dealt to
     // the XCDs round-robin instead.
-    const int L = VARLEN ? xcd_chunk_remap((int)blockIdx.x, total_units, units_per_bh * group)
+    // Teams: one query tile per workgroup, the heaviest tiles first; with a
+    // multiple of 8 slices a slice's tiles share an XCD.
+    const int L = SINGLE ? (int)blockIdx.x
+                : VARLEN ? xcd_chunk_remap((int)blockIdx.x, total_units, units_per_bh * group)
                          : xcd_remap((int)blockIdx.x, total_units);
-    const int bh = L / units_per_bh, u = L % units_per_bh;
-    const int b = bh / hq, h = bh - b * hq, hkv = hq / group, kvh = h / group;
+    int bh = L / units_per_bh, u = L - bh * units_per_bh;
+    if constexpr (SINGLE) {
+        const int first = L / (span * units_per_bh) * span, r = L - first * units_per_bh;
+        const int some = min(span, total_units / units_per_bh - first);
+        u = r / some;
+        bh = first + r - u * some;
+    }
+    const int hkv = hq / group, b = bh / hq;
+    int h = bh - b * hq;
+    if constexpr (SINGLE) h = h % hkv * group + h / hkv;  // the heads of a kv head hkv slices apart: on one XCD
+    const int kvh = h / group;
     int n, qs, ks;
     size_t qbase, kvbase;
     if (VARLEN) {
@@ -814,78 +887,190 @@ flash_prefill_kernel(const f16* __restrict__ Q, const f16* __restrict__ K, const
     } else {
         n = n_max;
         qs = ks = D;
-        qbase = (size_t)bh * n * D;
+        qbase = ((size_t)b * hq + h) * n * D;
         kvbase = ((size_t)b * hkv + kvh) * n * D;
     }
     const int nqt = (n + T::BM - 1) / T::BM;
-    if (VARLEN && u >= (CAUSAL ? (nqt + 1) / 2 : nqt)) return;  // whole workgroup: past this sequence
+    if (VARLEN && !SINGLE && u >= (CAUSAL ? (nqt + 1) / 2 : nqt)) return;  // whole workgroup: past this sequence
     const f16 *Qb = Q + qbase, *Kb = K + kvbase, *Vb = V + kvbase;
     f16* Ob = O + qbase;
-    if (CAUSAL) {
+    if constexpr (SINGLE) {
+        const int tile = units_per_bh - 1 - u;
+        if (VARLEN && tile >= nqt) return;
+        prefill_qtile<D, CAUSAL, NW, M, KG>(Qb, Kb, Vb, Ob, lds, tile * T::BM, n, qs, ks, sl2, qflip);
+    } else if (CAUSAL) {
         // Pair the heaviest remaining tile with the lightest: equal work per workgroup.
         const int heavy = nqt - 1 - u;
-        prefill_qtile<D, true, NW, M>(Qb, Kb, Vb, Ob, lds, heavy * T::BM, n, qs, ks, sl2, qflip);
+        prefill_qtile<D, true, NW, M, 1>(Qb, Kb, Vb, Ob, lds, heavy * T::BM, n, qs, ks, sl2, qflip);
         if (u != heavy) {
             __syncthreads();  // every wave is done with the buffers before they are refilled
-            prefill_qtile<D, true, NW, M>(Qb, Kb, Vb, Ob, lds, u * T::BM, n, qs, ks, sl2, qflip);
+            prefill_qtile<D, true, NW, M, 1>(Qb, Kb, Vb, Ob, lds, u * T::BM, n, qs, ks, sl2, qflip);
         }
     } else {
-        prefill_qtile<D, false, NW, M>(Qb, Kb, Vb, Ob, lds, u * T::BM, n, qs, ks, sl2, qflip);
+        prefill_qtile<D, false, NW, M, 1>(Qb, Kb, Vb, Ob, lds, u * T::BM, n, qs, ks, sl2, qflip);
     }
 }
 
-template <int D, bool CAUSAL, int NW, int M>
-static hipError_t launch_prefill_nw(const PrefillArgs& a) {
+// How a launch cuts its work; the numbers are MI355X us, 32x32x16 MFMAs unless
+// noted, "tiles" the 128-row query tiles of all slices.
+enum class PrefillKind {
+    kWaves4, kWaves8, kWaves8M16,  // NW waves, causal: query tiles in pairs of equal work
+    kSingle4, kSingle8, kSingle8M16,  // causal: one query tile per workgroup, the heaviest first
+    kTeams42, kTeams24, kTeams14,  // <waves><teams>: one query tile, its key tiles dealt to teams of waves
+};
+struct PrefillPlan {
+    PrefillKind kind;
+    int span;  // single tiles and teams: slices per group of workgroups
+};
+
+// Workgroup size where query tiles go in pairs (causal) or one by one.  8
+// waves (256 rows) share each K/V tile among more rows and win on long
+// sequences; 4 waves (128 rows, two workgroups per CU) halve the diagonal band
+// a causal workgroup pays in full and double the workgroup count, which wins
+// on short sequences and small grids.  Measured crossovers: causal up to N =
+// 2048 (+25% at 512, +5% at 2048, -4% at 8192), non-causal up to N = 1024
+// (+10% at 512, 0..+2% at 1024, -3..-6% beyond), and any grid of fewer 8-wave
+// workgroups than half the CUs.
+//
+// MFMA shape: 16x16x32 where the key loop is long enough for its lower energy
+// per FLOP (a higher clock under the power limit) to outweigh its twice as
+// many MFMA issues: D = 128, 8-wave workgroups, causal pairs from N = 6144,
+// non-causal from N = 3072.  Measured against 32x32x16 on one box at a time:
+// causal N = 8192 +0% to +4%, non-causal N = 4096 +4.5% to +6.7%, N = 3072
+// +1%, N = 2048 even; causal pairs at N = 3072-4096 -4% to -7%, the 4-wave
+// kernels -6% to -9%, and D = 64 -3% to -11% (its two exponentials per 32x32
+// MFMA leave no issue slots for the extra MFMA instructions).
+static PrefillKind prefill_full(int64_t n, int d, bool causal, int64_t bh) {
+    const int64_t nqt8 = (n + 255) / 256;
+    const int64_t wg8 = (causal ? (nqt8 + 1) / 2 : nqt8) * bh;
+    if (n <= (causal ? 2048 : 1024) || wg8 < 128) return PrefillKind::kWaves4;
+    return d == 128 && n >= (causal ? 6144 : 3072) ? PrefillKind::kWaves8M16 : PrefillKind::kWaves8;
+}
+
+// Teams while the grid is small.  A workgroup per CU of 8 waves then has
+// nobody to share the CU with, and its time is its longest chain of key tiles;
+// teams that take every second (or fourth) key tile of the same rows shorten
+// it, and smaller row tiles give more workgroups.  Each choice holds while its
+// workgroups fit one round of one per CU; causal grids, whose light tiles fill
+// in behind the heavy ones, hold further.  Measured, pairs or 4-wave workgroups
+// -> teams: non-causal N = 1024, 8 heads D = 64 15.0 -> 9.9 (14), D = 128 20.9
+// -> 15.1 (14); N = 4096, 4 heads, D = 64 48 -> 28 (24), 8 heads 60 -> 42 (42);
+// causal N = 256, 4 heads, D = 64 11.6 -> 6.3 (14), N = 2048, 8 heads, D = 64
+// 33.7 -> 16.6 (24), N = 8192, 8 heads, D = 128 199 -> 139 (42).  Short key
+// loops do not pay for the merge: the lower bounds on n.
+// D = 128 from 1025 to 3071 rows stays out: there every grid runs the same
+// MFMAs over the same key tiles in the same order, so that a head's result
+// does not depend on how many others run beside it; from 3072 rows the MFMA
+// shape of the large grids already differs.
+static bool prefill_teams(int64_t n, int d, bool causal, int64_t wg32, int64_t wg64, int64_t wg128, int64_t cus,
+                          PrefillKind& kind) {
+    if (d == 128 && n > 1024 && n < 3072) return false;
+    const bool d64 = d == 64;
+    if (wg32 <= cus && (d64 || (n <= 1024 && n >= (causal ? 96 : 192)))) kind = PrefillKind::kTeams14;
+    else if ((wg64 <= cus && n >= (causal ? 64 : d64 ? 640 : 768)) || (causal && wg128 <= cus && n >= 2048))
+        kind = PrefillKind::kTeams24;
+    else if (causal ? wg128 <= std::min(2 * cus, cus * n / 900) : wg128 <= cus && n >= 1536)
+        kind = PrefillKind::kTeams42;
+    else return false;
+    return true;
+}
+
+// Causal grids too large for teams.  One tile per workgroup, heaviest first,
+// fills the last round with light tiles and costs no idle slots where pairs
+// make a partial round; pairs keep two rules: three to four workgroups' worth
+// of 128-row tiles per CU up to N = 1024 (pairs then make exactly one round),
+// and long sequences on large grids (8-wave pairs 976 against 986 at 64 heads
+// x 8192, D = 128).  Measured, pairs -> single: D = 128 128 heads x 512 23.5 ->
+// 19.3, 512 x 512 82.6 -> 74.7, 40 x 2048 60.3 -> 53.0; with 16x16x32 MFMAs 32
+// heads x 4096 138 -> 132, 64 x 4096 288 -> 273; D = 64 128 heads x 700 25.4
+// -> 19.4, 256 x 1024 60.1 -> 57.0, 64 x 4096 170 -> 163.
+static PrefillKind prefill_causal(int64_t n, int d, int64_t bh, int64_t wg128, int64_t cus) {
+    if (d == 128 ? n < 3072 : n <= 3072)
+        return n <= 1024 && wg128 > 3 * cus && wg128 <= 4 * cus ? PrefillKind::kWaves4 : PrefillKind::kSingle4;
+    if (4 * wg128 <= 11 * cus) return PrefillKind::kSingle4;
+    if (d == 128 && (n <= 5120 || 2 * wg128 <= 7 * cus)) return PrefillKind::kSingle8M16;
+    if (d == 64 && n <= 4608) return 4 * wg128 <= 17 * cus ? PrefillKind::kSingle8 : PrefillKind::kSingle4;
+    return prefill_full(n, d, true, bh);
+}
+
+static PrefillPlan prefill_plan(const PrefillArgs& a) {
+    int dev = 0, cu_count = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cu_count, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu_count <= 0)
+        cu_count = 256;
+    const int64_t cus = cu_count, n = a.n;
+    // Workgroups that have rows, for row tiles of 32, 64 and 128 (packed
+    // sequences: at most so many, whatever their lengths).
+    auto tiles = [&](int64_t rows) {
+        return a.cu ? (a.total_rows / rows + a.bh / a.hq) * a.hq : (n + rows - 1) / rows * a.bh;
+    };
+    const int64_t wg128 = tiles(128);
+    PrefillPlan p{prefill_full(n, a.d, a.causal, a.bh), (int)a.bh};
+    if (prefill_teams(n, a.d, a.causal, tiles(32), tiles(64), wg128, cus, p.kind) || !a.causal) return p;
+    if ((n + 127) / 128 * a.bh > INT_MAX / 2) return p;  // twice the workgroups of the pairs
+    if (!a.cu) {
+        p.kind = prefill_causal(n, a.d, a.bh, wg128, cus);
+        // Groups of slices of about two workgroups per CU (8 waves: two rounds),
+        // 64 slices at most, so that the K and V read at a time, 8 * 4 MB over the XCDs, stay in
+        // their L2 (512 heads x 512, D = 128: 74.7 in groups of 64, 75.9 of 128, 85.0 in one);
+        // the same number in each group, a multiple of 8 (the XCDs).
+        const int64_t rows = p.kind == PrefillKind::kSingle4 ? 128 : 256, units = (n + rows - 1) / rows;
+        const int64_t some = std::min<int64_t>(64, std::max<int64_t>(8, 2 * cus / units));
+        const int64_t groups = std::max<int64_t>(1, a.bh / some);
+        p.span = (int)(((a.bh + groups - 1) / groups + 7) / 8 * 8);
+        return p;
+    }
+    // Packed sequences: single tiles also spread the long ones (12 of 64-4096
+    // tokens, 32 heads over 8, D = 128 1099 -> 991, D = 64 700 -> 588; 18 of
+    // 16-2080, 4 heads 74.6 -> 61.0); few long ones keep pairs (4 of up to 5000,
+    // 8 heads: 138 against 145).  Past 4608 rows 16x16x32 MFMAs (16 of 512-8192
+    // 4756 -> 4482).  Groups of whole sequences, of 32 slices or more, once the
+    // batch makes several rounds.
+    if (n > 2560 && wg128 < 8 * cus) return p;
+    p.kind = a.d == 64 || n <= 4608 ? PrefillKind::kSingle4 : PrefillKind::kSingle8M16;
+    if (wg128 > 10 * cus) p.span = (int)((31 + a.hq) / a.hq * a.hq);
+    return p;
+}
+
+template <int D, bool CAUSAL, int NW, int M, int KG = 1, bool SINGLE = false>
+static hipError_t launch_prefill_nw(const PrefillArgs& a, int span) {
     using T = PrefillTile<D, NW, M>;
     const int nqt = (int)((a.n + T::BM - 1) / T::BM);  // a.n: the (longest) sequence length
-    const int units = CAUSAL ? (nqt + 1) / 2 : nqt;
+    const int units = CAUSAL && !SINGLE ? (nqt + 1) / 2 : nqt;
     const long long total = (long long)units * a.bh;
     if (total <= 0) return hipSuccess;
     const int group = (int)(a.hq / a.hkv);
-    if (a.cu)
-        hipLaunchKernelGGL((flash_prefill_kernel<D, CAUSAL, true, NW, M>), dim3((unsigned)total), dim3(T::THREADS), 0,
-                           (hipStream_t)a.stream, (const f16*)a.q, (const f16*)a.k, (const f16*)a.v, (f16*)a.o,
-                           a.cu, (int)a.total_rows, (int)a.n, units, (int)total, (int)a.hq, group, a.sl2, a.qflip);
-    else
-        hipLaunchKernelGGL((flash_prefill_kernel<D, CAUSAL, false, NW, M>), dim3((unsigned)total), dim3(T::THREADS), 0,
-                           (hipStream_t)a.stream, (const f16*)a.q, (const f16*)a.k, (const f16*)a.v, (f16*)a.o,
-                           a.cu, 0, (int)a.n, units, (int)total, (int)a.hq, group, a.sl2, a.qflip);
+    auto launch = [&](auto* kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(T::THREADS * KG), 0, (hipStream_t)a.stream,
+                           (const f16*)a.q, (const f16*)a.k, (const f16*)a.v, (f16*)a.o, a.cu, (int)a.total_rows,
+                           (int)a.n, units, (int)total, span, (int)a.hq, group, a.sl2, a.qflip);
+    };
+    if (a.cu) launch(flash_prefill_kernel<D, CAUSAL, true, NW, M, KG, SINGLE>);
+    else launch(flash_prefill_kernel<D, CAUSAL, false, NW, M, KG, SINGLE>);
     return hipGetLastError();
-}
-
-// Workgroup size.  8 waves (256 rows) share each K/V tile among more rows and
-// win on long sequences; 4 waves (128 rows, two workgroups per CU) halve the
-// diagonal band a causal workgroup pays in full and double the workgroup count,
-// which wins on short sequences and small grids.  Measured crossovers on
-// MI355X: causal up to N = 2048 (+25% at 512, +5% at 2048, -4% at 8192),
-// non-causal up to N = 1024 (+10% at 512, 0..+2% at 1024, -3..-6% beyond), and
-// any grid of fewer 8-wave workgroups than half the CUs.
-static int prefill_waves(int64_t n, bool causal, int64_t bh) {
-    const int64_t nqt8 = (n + 255) / 256;
-    const int64_t wg8 = (causal ? (nqt8 + 1) / 2 : nqt8) * bh;
-    if (n <= (causal ? 2048 : 1024) || wg8 < 128) return 4;
-    return 8;
-}
-
-// MFMA shape.  16x16x32 where the key loop is long enough for its lower energy
-// per FLOP (a higher clock under the power limit) to outweigh its twice as
-// many MFMA issues: D = 128, 8-wave workgroups, causal N >= 6144, non-causal
-// N >= 3072.  Measured against 32x32x16 on one box at a time: causal N = 8192
-// +0% to +4%, non-causal N = 4096 +4.5% to +6.7%, N = 3072 +1%, N = 2048 even;
-// causal N = 3072-4096 -4% to -7%, the 4-wave kernels -6% to -9%, and D = 64
-// -3% to -11% (its two exponentials per 32x32 MFMA leave no issue slots for
-// the extra MFMA instructions).
-static bool prefill_mfma16(int64_t n, int d, int nw, bool causal) {
-    return d == 128 && nw == 8 && n >= (causal ? 6144 : 3072);
 }
 
 template <int D, bool CAUSAL>
 static hipError_t launch_prefill(const PrefillArgs& a) {
-    if (prefill_waves(a.n, CAUSAL, a.bh) == 4) return launch_prefill_nw<D, CAUSAL, 4, 32>(a);
-    if constexpr (D == 128) {
-        if (prefill_mfma16(a.n, D, 8, CAUSAL)) return launch_prefill_nw<D, CAUSAL, 8, 16>(a);
+    const PrefillPlan p = prefill_plan(a);
+    switch (p.kind) {
+        case PrefillKind::kTeams42: return launch_prefill_nw<D, CAUSAL, 4, 32, 2, true>(a, p.span);
+        case PrefillKind::kTeams24: return launch_prefill_nw<D, CAUSAL, 2, 32, 4, true>(a, p.span);
+        case PrefillKind::kTeams14: return launch_prefill_nw<D, CAUSAL, 1, 32, 4, true>(a, p.span);
+        case PrefillKind::kWaves4: return launch_prefill_nw<D, CAUSAL, 4, 32>(a, p.span);
+        case PrefillKind::kWaves8: return launch_prefill_nw<D, CAUSAL, 8, 32>(a, p.span);
+        default: break;
     }
-    return launch_prefill_nw<D, CAUSAL, 8, 32>(a);
+    if constexpr (CAUSAL) {
+        if (p.kind == PrefillKind::kSingle4) return launch_prefill_nw<D, true, 4, 32, 1, true>(a, p.span);
+        if constexpr (D == 64)
+            if (p.kind == PrefillKind::kSingle8) return launch_prefill_nw<D, true, 8, 32, 1, true>(a, p.span);
+        if constexpr (D == 128)
+            if (p.kind == PrefillKind::kSingle8M16) return launch_prefill_nw<D, true, 8, 16, 1, true>(a, p.span);
+    }
+    if constexpr (D == 128)
+        if (p.kind == PrefillKind::kWaves8M16) return launch_prefill_nw<D, CAUSAL, 8, 16>(a, p.span);
+    return hipErrorInvalidValue;
 }
 
 hipError_t prefill_launch(const PrefillArgs& a) {

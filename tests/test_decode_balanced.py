@@ -18,6 +18,7 @@ BATCHES = {
     "two": [1, 4099],
     "empty": [0, 1500, 0, 2049, 0],                  # outside the >= 1 contract: zero rows
 }
+LONGEST = 1 << 16  # max_context_len given, so that even the small batches are cut by the kernel
 
 
 @pytest.mark.parametrize("name", BATCHES)
@@ -33,20 +34,20 @@ def test_matches_oracle(name, g, hkv, d, bs):
     ref = np.zeros(q.shape, np.float32)
     ref[rows] = oracle.paged_decode_fp32(q[rows], kc, vc, bt[rows], cl[rows])
     for _ in range(2):
-        assert max_err(ak.paged_decode(*dev, max(lens)), ref) < TOL[d]
+        assert max_err(ak.paged_decode(*dev, LONGEST), ref) < TOL[d]
     # other lengths right after, on the same counters
     dev[4] = torch.clamp(dev[4] // 2, min=1)
     short = cl // 2
     short[short < 1] = 1
-    assert max_err(ak.paged_decode(*dev, max(lens)), oracle.paged_decode_fp32(q, kc, vc, bt, short)) < TOL[d]
+    assert max_err(ak.paged_decode(*dev, LONGEST), oracle.paged_decode_fp32(q, kc, vc, bt, short)) < TOL[d]
 
 
 def test_tokens_past_the_longest_context_given_are_cut_as_with_fixed_splits():
     """A length above max_context_len (outside the contract) reads up to the end of the last fixed split."""
-    kc, vc, bt, cl = oracle.make_paged_cache([6000, 300], 2, 128, block_size=16, extra_blocks=1, seed=1)
+    kc, vc, bt, cl = oracle.make_paged_cache([20000, 300], 4, 128, block_size=16, extra_blocks=1, seed=1)
     q = np.random.default_rng(2).standard_normal((2, 8, 128), dtype=np.float32).astype(np.float16)
     dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, bt, cl)]
-    part = ak.decode_partition(2, 2, 3000)
-    a = ak.paged_decode(*dev, 3000)
-    b = ak.paged_decode(*dev, 3000, partition_size=part)
+    part = ak.decode_partition(2, 4, 16500)
+    a = ak.paged_decode(*dev, 16500)
+    b = ak.paged_decode(*dev, 16500, partition_size=part)
     assert max_err(a, b.float().cpu().numpy()) < 1e-3

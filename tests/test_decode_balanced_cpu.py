@@ -106,8 +106,8 @@ def workers(lib, batch, hq, hkv, d, max_ctx, partition=1024):
 
 
 def test_rule(lib):
-    # fixed splits: one sequence, more than 64, short contexts, lengths past 2^24, invalid sizes
-    for args in ((1, 32, 8, 128, 8192), (65, 32, 8, 128, 8192), (16, 32, 8, 128, 1024), (16, 32, 8, 128, 1 << 24),
+    # fixed splits: one sequence, more than 64, short contexts, little K and V, lengths past 2^24, invalid sizes
+    for args in ((1, 32, 8, 128, 8192), (65, 32, 8, 128, 8192), (16, 32, 8, 128, 1024), (16, 32, 8, 128, 1 << 24), (3, 16, 4, 128, 8100),
                  (16, 32, 0, 128, 8192), (16, 30, 8, 128, 8192), (0, 32, 8, 128, 8192)):
         assert workers(lib, *args) == 0, args
     assert workers(lib, 16, 32, 8, 128, 8192, 0) == 0
@@ -117,6 +117,9 @@ def test_rule(lib):
             for d in (64, 128):
                 for ctx in (1025, 8192, 8193, 100000):
                     w = workers(lib, batch, hq, hkv, d, ctx)
+                    if batch * hkv * ctx * d * 4 < 64 << 20:
+                        assert w == 0
+                        continue
                     if w == 0:  # no room to cut: about one workgroup per sequence
                         assert hq == hkv and d == 128 and ctx <= 8192
                         continue

@@ -111,6 +111,39 @@ def test_mfma_shape_boundaries(causal, h, n):
         assert max_err(out[:, hi], ref) < TOL[128], hi
 
 
+@pytest.mark.parametrize("d,causal,h,n", [
+    # teams of one wave x 4, two x 4 and four x 2: tiles without keys for a team, ragged row and key tiles
+    (64, False, 8, 257), (128, True, 4, 97), (64, True, 3, 65), (64, False, 5, 1537), (128, False, 10, 801),
+    (64, True, 6, 2049), (128, True, 6, 3073), (64, False, 14, 2047), (64, True, 30, 1023), (128, False, 8, 3073),
+    (128, True, 12, 3100), (64, True, 300, 1),
+    # single tiles: one group of slices, several with a smaller last one, 8 waves, 16x16 MFMAs
+    (128, True, 64, 700), (64, True, 70, 385), (128, True, 520, 257), (64, True, 24, 4097), (128, True, 26, 3585),
+    # pairs between three and four workgroups' worth of tiles per CU
+    (128, True, 200, 513)])
+def test_work_splits(d, causal, h, n):
+    """Each way a launch cuts its work, at sizes with remainders: first, a middle and last head against the oracle."""
+    print(f"work split d={d} causal={causal} h={h} n={n}", flush=True)
+    q, k, v = rand_qkv(1, h, n, d, seed=n + h)
+    out = run("wmma64", q, k, v, causal)
+    assert torch.isfinite(out).all()
+    for hi in (0, h // 2, h - 1):
+        ref = oracle.attention_fp32(q[:, hi].numpy(), k[:, hi].numpy(), v[:, hi].numpy(), causal)
+        assert max_err(out[:, hi], ref) < TOL[d], hi
+
+
+def test_teams_when_the_maximum_sits_in_one_teams_keys():
+    """Teams of very different maxima (keys 64-127 score far above the rest), and
+    causal rows that see none of a team's keys: the merge weighs them."""
+    for d, n in ((64, 200), (128, 200), (64, 2100)):
+        q, k, v = rand_qkv(1, 2, n, d, seed=21)
+        k[:, :, 64:128] *= 8
+        for causal in (False, True):
+            out = run("wmma64", q, k, v, causal)
+            assert torch.isfinite(out).all()
+            ref = oracle.attention_fp32(q.numpy(), k.numpy(), v.numpy(), causal)
+            assert max_err(out, ref) < 2 * TOL[d]
+
+
 def test_causal_first_row_is_v0():
     q, k, v = rand_qkv(1, 1, 128, 64, seed=5)
     for name in VARIANTS:

@@ -56,7 +56,8 @@ def packed(lens, h, hkv, d, seed=0):
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("lens,h,hkv", [([1, 255, 256, 257, 3], 4, 4), ([700, 40, 1300], 8, 2),
-                                        ([129, 0, 511, 64], 6, 3)])
+                                        ([129, 0, 511, 64], 6, 3), ([33, 800, 0, 5], 4, 2),
+                                        ([5] * 70 + [300], 16, 4)])
 def test_varlen_matches_oracle(d, causal, lens, h, hkv):
     q, k, v, cu = packed(lens, h, hkv, d, seed=sum(lens))
     out = ak.flash_attention_varlen(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), max(lens), causal=causal)
