@@ -957,17 +957,19 @@ static PrefillKind prefill_full(int64_t n, int d, bool causal, int64_t bh) {
 // -> 15.1 (14); N = 4096, 4 heads, D = 64 48 -> 28 (24), 8 heads 60 -> 42 (42);
 // causal N = 256, 4 heads, D = 64 11.6 -> 6.3 (14), N = 2048, 8 heads, D = 64
 // 33.7 -> 16.6 (24), N = 8192, 8 heads, D = 128 199 -> 139 (42).  Short key
-// loops do not pay for the merge: the lower bounds on n.
+// loops do not pay for the merge: the lower bounds on n (16 heads x 160, D = 128
+// causal: 7.8 in single tiles, 8.7-9.0 in teams; 32 heads x 300, D = 64: 7.7
+// against 8.1 with two waves by four).
 // D = 128 from 1025 to 3071 rows stays out: there every grid runs the same
 // MFMAs over the same key tiles in the same order, so that a head's result
 // does not depend on how many others run beside it; from 3072 rows the MFMA
 // shape of the large grids already differs.
 static bool prefill_teams(int64_t n, int d, bool causal, int64_t wg32, int64_t wg64, int64_t wg128, int64_t cus,
                           PrefillKind& kind) {
-    if (d == 128 && n > 1024 && n < 3072) return false;
+    if (n <= 192 || (d == 128 && n > 1024 && n < 3072)) return false;
     const bool d64 = d == 64;
-    if (wg32 <= cus && (d64 || (n <= 1024 && n >= (causal ? 96 : 192)))) kind = PrefillKind::kTeams14;
-    else if ((wg64 <= cus && n >= (causal ? 64 : d64 ? 640 : 768)) || (causal && wg128 <= cus && n >= 2048))
+    if (wg32 <= cus && (d64 || n <= 1024)) kind = PrefillKind::kTeams14;
+    else if ((wg64 <= cus && n > (causal ? 320 : d64 ? 640 : 768)) || (causal && wg128 <= cus && n >= 2048))
         kind = PrefillKind::kTeams24;
     else if (causal ? wg128 <= std::min(2 * cus, cus * n / 900) : wg128 <= cus && n >= 1536)
         kind = PrefillKind::kTeams42;
@@ -985,6 +987,7 @@ static bool prefill_teams(int64_t n, int d, bool causal, int64_t wg32, int64_t w
 // heads x 4096 138 -> 132, 64 x 4096 288 -> 273; D = 64 128 heads x 700 25.4
 // -> 19.4, 256 x 1024 60.1 -> 57.0, 64 x 4096 170 -> 163.
 static PrefillKind prefill_causal(int64_t n, int d, int64_t bh, int64_t wg128, int64_t cus) {
+    if (n <= 128) return PrefillKind::kWaves4;  // one tile: the pairs' index arithmetic is shorter (0.1 us)
     if (d == 128 ? n < 3072 : n <= 3072)
         return n <= 1024 && wg128 > 3 * cus && wg128 <= 4 * cus ? PrefillKind::kWaves4 : PrefillKind::kSingle4;
     if (4 * wg128 <= 11 * cus) return PrefillKind::kSingle4;
@@ -1010,12 +1013,15 @@ static PrefillPlan prefill_plan(const PrefillArgs& a) {
     if ((n + 127) / 128 * a.bh > INT_MAX / 2) return p;  // twice the workgroups of the pairs
     if (!a.cu) {
         p.kind = prefill_causal(n, a.d, a.bh, wg128, cus);
-        // Groups of slices of about two workgroups per CU (8 waves: two rounds),
-        // 64 slices at most, so that the K and V read at a time, 8 * 4 MB over the XCDs, stay in
-        // their L2 (512 heads x 512, D = 128: 74.7 in groups of 64, 75.9 of 128, 85.0 in one);
-        // the same number in each group, a multiple of 8 (the XCDs).
+        // Groups of slices once their K and V no longer fit the XCDs' L2 (8 * 4 MB;
+        // 256 heads x 220, D = 64, 29 MB: 9.5 in one group, 10.9 in groups of 64):
+        // about two workgroups per CU (8 waves: two rounds), or one per CU if
+        // that is 64 slices or more (512 heads x 512, D = 128: 74.7 in groups of
+        // 64, 75.9 of 128, 85.0 in one); the same number in each group, a
+        // multiple of 8 (the XCDs).
+        if (a.bh / a.hq * a.hkv * n * a.d * 4 <= int64_t(32) << 20) return p;
         const int64_t rows = p.kind == PrefillKind::kSingle4 ? 128 : 256, units = (n + rows - 1) / rows;
-        const int64_t some = std::min<int64_t>(64, std::max<int64_t>(8, 2 * cus / units));
+        const int64_t some = std::max<int64_t>(8, std::min(std::max<int64_t>(64, cus / units), 2 * cus / units));
         const int64_t groups = std::max<int64_t>(1, a.bh / some);
         p.span = (int)(((a.bh + groups - 1) / groups + 7) / 8 * 8);
         return p;
