@@ -319,13 +319,13 @@ __device__ __forceinline__ float dot8(f16x8 a, f16x8 b) {
     return s;
 }
 
-template <int D>
+template <int D, bool BALANCED>
 __global__ void __launch_bounds__((DecodeTile<D>::THREADS))
 paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const f16* __restrict__ vc,
                     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
                     f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                     float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs, int bs_shift,
-                    int max_blocks, int num_blocks, int partition, int num_splits, float sl2, int balanced, int batch,
+                    int max_blocks, int num_blocks, int partition, int num_splits, float sl2, int batch,
                     int cap) {
     using T = DecodeTile<D>;
     constexpr int G = 1;
@@ -339,10 +339,10 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;  // never index past the table row
-    const Segment sg = balanced ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
-    if (b < 0) return;
+    if (BALANCED && b < 0) return;
     const int* bt = block_tables + (size_t)b * max_blocks;
 
     // Page ids of this lane's tokens in the chunk starting at t0, for tokens
@@ -594,14 +594,14 @@ __device__ __forceinline__ float across_groups(float x, Op op) {
     return xor_combine<32>(x, op);
 }
 
-template <int D, int G, int NW, bool PIPE>
+template <int D, int G, int NW, bool PIPE, bool BALANCED>
 __global__ void __launch_bounds__((GqaTile<D, G, NW>::THREADS))
 paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const f16* __restrict__ vc,
                         const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
                         f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                         float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                         int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits, float sl2,
-                        int balance, int balanced, int batch, int cap) {
+                        int balance, int batch, int cap) {
     using T = GqaTile<D, G, NW>;
     constexpr int U = T::U, N = T::N, S = T::S, LB = T::LB;
     // P = 2^(s - m + kPShift): the largest P the fast path accepts is 2^kPMax.
@@ -614,10 +614,10 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;
-    const Segment sg = balanced ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
-    if (b < 0) return;
+    if (BALANCED && b < 0) return;
     const int* bt = block_tables + (size_t)b * max_blocks;
 
     // Value index of a partial dot product: j = (slot >> 1) * 2G + head * 2 +
@@ -930,14 +930,14 @@ struct GqaMfmaTile {
 // At most 168 VGPRs (amdgpu_waves_per_eu(3)), so that three waves share a
 // SIMD (the compiler otherwise moves the accumulators to AGPRs and holds 172
 // registers, two waves); a 128-register bound spills at D = 128.
-template <int D, int G, int NW>
+template <int D, int G, int NW, bool BALANCED>
 __global__ void __launch_bounds__((GqaMfmaTile<D, G, NW>::THREADS)) __attribute__((amdgpu_waves_per_eu(3)))
 paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const f16* __restrict__ vc,
                              const int* __restrict__ block_tables, const int* __restrict__ ctx_lens,
                              f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                              float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                              int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits,
-                             float sl2, int balance, int balanced, int batch, int cap) {
+                             float sl2, int balance, int batch, int cap) {
     using T = GqaMfmaTile<D, G, NW>;
     constexpr int KS = T::KS, DPL = T::DPL;
     typedef _Float16 vrow_t __attribute__((ext_vector_type(DPL)));
@@ -951,10 +951,10 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int max_tok = max_blocks * bs;
-    const Segment sg = balanced ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
-    if (b < 0) return;
+    if (BALANCED && b < 0) return;
     const int* bt = block_tables + (size_t)b * max_blocks;
     const int stride = NW * T::TOK;
     const bool fast_bs = bs == 16;
@@ -1340,39 +1340,44 @@ static hipError_t launch_decode(const DecodeArgs& a) {
         hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, stream, (const f16*)a.q, (const f16*)a.k_cache,
                            (const f16*)a.v_cache, a.block_tables, a.context_lens, (f16*)a.out, a.o_part, a.m_part,
                            a.l_part, counters, (int)a.hkv, (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks,
-                           (int)a.partition, (int)a.num_splits, a.sl2, more..., (int)a.balanced, (int)a.batch,
+                           (int)a.partition, (int)a.num_splits, a.sl2, more..., (int)a.batch,
                            (int)a.token_cap);
     };
-    if constexpr (G == 1) {
-        launch(paged_decode_kernel<D>, DecodeTile<D>::THREADS);
-    } else {
-        const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
-        auto launch_nw = [&](auto nw) {
-            constexpr int NW = decltype(nw)::value;
-            if constexpr (G == 8) {
-                constexpr auto K = paged_decode_gqa_mfma_kernel<D, G, NW>;
-                launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
-            } else {
-                constexpr auto K = paged_decode_gqa_kernel<D, G, NW, gqa_pipelined(D, G)>;
-                launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
-            }
-        };
-        // Waves per workgroup of both grouped-query kernels.  A dot-product wave
-        // reads one 16-token page per round trip to memory, so a split of P tokens
-        // costs P / (16 NW) dependent round trips; with many workgroups per CU they
-        // overlap, but in a small grid (one sequence, few kv heads) they are the
-        // kernel's critical path.  Measured on MI355X (one call after a 512 MiB flush,
-        // G = 2, 4, 8, D = 64 and 128): grids under 512 workgroups run 0.3-1.9 us
-        // faster with 8 waves than with 4 (B=1 ctx 1024: 11.8 vs 13.7 us; ctx 16384:
-        // 20.8 vs 21.4 us), and 16 waves are slower than 8 everywhere; from 512
-        // workgroups up, 4 waves win.  The matrix-core kernel (two pages per round
-        // trip) measured the same way picks the same: 4 waves at B = 8 x 8192 tokens
-        // (8 waves -2%), 8 at B = 1 (equal or better).
-        if (wgs * 4 >= kGqaManyWaves)
-            launch_nw(std::integral_constant<int, 4>{});
-        else
-            launch_nw(std::integral_constant<int, 8>{});
-    }
+    auto launch_mode = [&](auto mode) {
+        constexpr bool BALANCED = decltype(mode)::value;
+        if constexpr (G == 1) {
+            launch(paged_decode_kernel<D, BALANCED>, DecodeTile<D>::THREADS);
+        } else {
+            const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+            auto launch_nw = [&](auto nw) {
+                constexpr int NW = decltype(nw)::value;
+                if constexpr (G == 8) {
+                    constexpr auto K = paged_decode_gqa_mfma_kernel<D, G, NW, BALANCED>;
+                    launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
+                } else {
+                    constexpr auto K = paged_decode_gqa_kernel<D, G, NW, gqa_pipelined(D, G), BALANCED>;
+                    launch(K, NW * kWave, (int)one_round<K>(NW * kWave, wgs));
+                }
+            };
+            // Waves per workgroup of both grouped-query kernels.  A dot-product wave
+            // reads one 16-token page per round trip to memory, so a split of P tokens
+            // costs P / (16 NW) dependent round trips; with many workgroups per CU they
+            // overlap, but in a small grid (one sequence, few kv heads) they are the
+            // kernel's critical path.  Measured on MI355X (one call after a 512 MiB flush,
+            // G = 2, 4, 8, D = 64 and 128): grids under 512 workgroups run 0.3-1.9 us
+            // faster with 8 waves than with 4 (B=1 ctx 1024: 11.8 vs 13.7 us; ctx 16384:
+            // 20.8 vs 21.4 us), and 16 waves are slower than 8 everywhere; from 512
+            // workgroups up, 4 waves win.  The matrix-core kernel (two pages per round
+            // trip) measured the same way picks the same: 4 waves at B = 8 x 8192 tokens
+            // (8 waves -2%), 8 at B = 1 (equal or better).
+            if (wgs * 4 >= kGqaManyWaves)
+                launch_nw(std::integral_constant<int, 4>{});
+            else
+                launch_nw(std::integral_constant<int, 8>{});
+        }
+    };
+    if (a.balanced) launch_mode(std::true_type{});
+    else launch_mode(std::false_type{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.num_splits == 1 || counters) return e;
     hipLaunchKernelGGL((paged_reduce_kernel<D>), dim3((unsigned)(a.batch * a.hq)), dim3(256), 0, stream,
