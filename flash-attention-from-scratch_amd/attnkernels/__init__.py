@@ -55,6 +55,13 @@ def load_extension():
     return mod
 
 
+def _on_gpu(x):
+    """Whether a call can be the plain one that the extension checks and runs in
+    one pass (its plain_* functions: None if it is not, and the checks and
+    conversions here follow)."""
+    return getattr(x, "is_cuda", False)
+
+
 def _check_prefill(q, k, v):
     """Reference attnkernels/__init__.py:53-61 (same checks, same ValueErrors)."""
     for t in (q, k, v):
@@ -85,6 +92,10 @@ def flash_attention(q, k, v, causal=False, scale=None, variant="wmma", block_n=N
     block_n: key-tile width accepted by "wmma" (32 or 64), as in the reference.
     Reference: attnkernels/__init__.py:71-85.
     """
+    if variant == "wmma" and block_n is None and _on_gpu(q):
+        out = load_extension().plain_prefill(q, k, v, causal, scale, False)
+        if out is not None:
+            return out
     q, k, v = _check_prefill(q, k, v)
     scale = 1.0 / math.sqrt(q.shape[-1]) if scale is None else scale
     ext = load_extension()
@@ -201,6 +212,11 @@ def paged_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_le
                   64, contexts up to 1024 tokens, less than 64 MB of K and V
                   at max_context_len), decode_partition picks one.
     """
+    if _on_gpu(q):
+        out = load_extension().plain_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_len, scale,
+                                            partition_size, decode_partition)
+        if out is not None:
+            return out
     if not (q.dtype == k_cache.dtype == v_cache.dtype == torch.float16):
         raise ValueError("q and caches must be fp16")
     if q.shape[-1] not in (64, 128) or k_cache.shape[-1] != q.shape[-1]:
@@ -225,6 +241,10 @@ def flash_attention_gqa(q, k, v, causal=False, scale=None):
     N, D] fp16 with H a multiple of H_kv; query head h reads kv head
     h // (H / H_kv).  Same kernel as ``flash_attention``, which (like the
     reference, attnkernels/__init__.py:57-58) requires H_kv == H."""
+    if _on_gpu(q):
+        out = load_extension().plain_prefill(q, k, v, causal, scale, True)
+        if out is not None:
+            return out
     for t in (q, k, v):
         if not (t.is_cuda and t.dtype == torch.float16 and t.dim() == 4):
             raise ValueError("q, k, v must be fp16 CUDA tensors of shape [B, H, N, D]")
@@ -248,6 +268,10 @@ def flash_attention_varlen(q, k, v, cu_seqlens, max_seqlen, causal=False, scale=
     host cu_seqlens is checked here; a device one is used as given (no sync):
     inconsistent offsets then give wrong rows, never an out-of-bounds access.
     """
+    if _on_gpu(q):
+        out = load_extension().plain_varlen(q, k, v, cu_seqlens, max_seqlen, causal, scale)
+        if out is not None:
+            return out
     for t in (q, k, v):
         if not (t.is_cuda and t.dtype == torch.float16 and t.dim() == 3):
             raise ValueError("q, k, v must be fp16 CUDA tensors of shape [total, H, D]")
@@ -286,6 +310,8 @@ def reshape_and_cache(key, value, k_cache, v_cache, slot_mapping):
                   row slot % block_size.  Negative slots (padding) and slots
                   past the pool are skipped.
     """
+    if _on_gpu(key) and load_extension().plain_write(key, value, k_cache, v_cache, slot_mapping):
+        return
     if key.dim() != 3 or value.shape != key.shape:
         raise ValueError("key and value must be [num_tokens, H_kv, D] of the same shape")
     if key.dtype not in (torch.float16, torch.bfloat16) or not (
