@@ -60,6 +60,18 @@ def test_strided_rows_from_fused_projection():
     _check(key, value, kc0, vc0, kc, vc, slots)
 
 
+@pytest.mark.parametrize("d", [40, 64, 128])
+@pytest.mark.parametrize("skip", [(), (0,), (1,), (0, 1), (8,), (2, 7, 8)])
+def test_odd_token_counts_and_skipped_halves_of_a_pair(d, skip):
+    """A workgroup moves two tokens: the last alone, either one skipped, or both."""
+    key, value, kc, vc, slots = _case(9, 5, d, 6, 8, torch.float16, seed=d)
+    slots[list(skip)] = -1
+    kc0, vc0 = kc.clone(), vc.clone()
+    ak.reshape_and_cache(key, value, kc, vc, slots)
+    torch.cuda.synchronize()
+    _check(key, value, kc0, vc0, kc, vc, slots)
+
+
 def test_padding_and_out_of_pool_slots_are_skipped():
     key, value, kc, vc, _ = _case(6, 8, 64, 4, 16, torch.float16, seed=3)
     slots = torch.tensor([5, -1, 63, 64, 1 << 40, 0], device="cuda", dtype=torch.int64)
