@@ -197,9 +197,11 @@ __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_
         incl = wave_scan(n);
         const int count = __builtin_amdgcn_readlane(incl, 63);
         if (count <= workers) break;
-        size = it < 6 ? round_up(size + 1 + (int)((float)size * (float)(count - workers) *
-                                                  __builtin_amdgcn_rcpf((float)workers)))
-                      : round_up(cap);  // one split per sequence: batch <= workers
+        // Uneven sequences have about total / size + batch / 2 splits.
+        const int more = it == 0 ? (int)((float)total * __builtin_amdgcn_rcpf((float)max(1, workers - batch / 2)))
+                                 : size + (int)((float)size * (float)(count - workers) *
+                                                __builtin_amdgcn_rcpf((float)workers));
+        size = it < 6 ? round_up(max(size, more) + 1) : round_up(cap);  // at last one split each: batch <= workers
     }
     const int j = blockIdx.y;
     Segment sg;
@@ -647,7 +649,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     };
     const int stride = T::NW * T::TOK;
     int pg[U];
-    const bool fast_bs = bs == T::TOK;
+    const bool fast_bs = bs_shift >= 4;  // pages of whole 16-token chunks
 
     if (start >= end) {
         if (num_splits == 1 || (counters && split == 0))
@@ -661,7 +663,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     // faster, uniform batches unchanged).
     int spg = 0;
     if (fast_bs && start + w * T::TOK + T::TOK <= end)
-        spg = bt[uniform((start + w * T::TOK) >> 4)];
+        spg = bt[uniform((start + w * T::TOK) >> bs_shift)];
     f16x8 qv[G];  // register a: query head a ^ fh
 #pragma unroll
     for (int a = 0; a < G; ++a)
@@ -774,20 +776,22 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
             }
         }
     };
-    // Byte offset of slot u's 16 bytes inside a 16-token page of this kv head.
+    // Byte offset of slot u's 16 bytes from the first row of a chunk.
     uint32_t lane_off[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-        lane_off[u] = (uint32_t)(((size_t)kvh * T::TOK * D + ((u ^ fu) * T::TPL + gi) * D + li * 8) * sizeof(f16));
+    for (int u = 0; u < U; ++u) lane_off[u] = (uint32_t)((((u ^ fu) * T::TPL + gi) * D + li * 8) * sizeof(f16));
+    const f16 *kch = kc + (size_t)kvh * bs * D, *vch = vc + (size_t)kvh * bs * D;  // this kv head of page 0
 
-    // Whole-page chunks: the chunk's page id is one wave-uniform scalar load
-    // (prefetched one chunk ahead) and every K/V load is page base + lane
-    // offset.  The checked loop takes the rest: the context's tail, an
-    // out-of-range page id, and every chunk when pages are not 16 tokens.
+    // Chunks in one page (a power of two of at least 16 tokens): the page id is
+    // one wave-uniform scalar load (prefetched one chunk ahead) and every K/V
+    // load is chunk base + lane offset.  The checked loop takes the rest: the
+    // context's tail, an out-of-range page id, and every chunk of other pages.
+    // Pages of 32 tokens went through the checked loop before: 16 sequences of
+    // 512-8192 tokens, Hq=32, 68.9 -> 54.1 us a call on MI355X, Hq=64 138 -> 60.
     int t0 = start + w * T::TOK;
     {
-        auto load_kv = [&](const f16* cache, int pid, f16x8 (&r)[U]) {
-            const char* base = reinterpret_cast<const char*>(cache) + (size_t)pid * page_stride * sizeof(f16);
+        auto load_kv = [&](const f16* cache, int pid, int t, f16x8 (&r)[U]) {
+            const char* base = reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + (t & (bs - 1)) * D);
 #pragma unroll
             for (int u = 0; u < U; ++u)  // streamed once: non-temporal
                 r[u] = __builtin_nontemporal_load(reinterpret_cast<const f16x8*>(base + lane_off[u]));
@@ -804,10 +808,10 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
                 const int tn = t0 + stride;
                 const bool issued = tn + T::TOK <= end && (unsigned)spn < (unsigned)num_blocks;
                 if (issued) {
-                    load_kv(kc, spn, knext);
-                    load_kv(vc, spn, vnext);
+                    load_kv(kch, spn, tn, knext);
+                    load_kv(vch, spn, tn, vnext);
                     const int tnn = tn + stride;
-                    if (tnn + T::TOK <= end) spn = bt[uniform(tnn >> 4)];
+                    if (tnn + T::TOK <= end) spn = bt[uniform(tnn >> bs_shift)];
                 }
                 if (balance) progress_priority(t0 - start, end - start);
                 float x[2];
@@ -818,20 +822,20 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
             };
             if (fast_bs && t0 + T::TOK <= end && (unsigned)spg < (unsigned)num_blocks) {
                 f16x8 ka[U], va[U], kb[U], vb[U];
-                load_kv(kc, spg, ka);
-                load_kv(vc, spg, va);
+                load_kv(kch, spg, t0, ka);
+                load_kv(vch, spg, t0, va);
                 int spn = -1;
-                if (t0 + stride + T::TOK <= end) spn = bt[uniform((t0 + stride) >> 4)];
+                if (t0 + stride + T::TOK <= end) spn = bt[uniform((t0 + stride) >> bs_shift)];
                 while (step(ka, va, kb, vb, spn) && step(kb, vb, ka, va, spn)) {
                 }
             }
         } else {
             while (fast_bs && t0 + T::TOK <= end && (unsigned)spg < (unsigned)num_blocks) {
                 f16x8 kr[U], vr[U];
-                load_kv(kc, spg, kr);
-                load_kv(vc, spg, vr);
+                load_kv(kch, spg, t0, kr);
+                load_kv(vch, spg, t0, vr);
                 const int tn = t0 + stride;
-                if (tn + T::TOK <= end) spg = bt[uniform(tn >> 4)];
+                if (tn + T::TOK <= end) spg = bt[uniform(tn >> bs_shift)];
                 if (balance) progress_priority(t0 - start, end - start);
                 float x[2];
                 scores(kr, x);
@@ -957,7 +961,7 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     if (BALANCED && b < 0) return;
     const int* bt = block_tables + (size_t)b * max_blocks;
     const int stride = NW * T::TOK;
-    const bool fast_bs = bs == 16;
+    const bool fast_bs = bs_shift >= 4;  // pages of whole 16-token chunks
     int t0 = start + w * T::TOK;
 
     if (start >= end) {
@@ -971,8 +975,8 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     // batch's grid) exits after its one scalar load.
     int spa = -1, spb = -1;  // page ids of the pair at t0 (wave-uniform), loaded one pair ahead
     if (fast_bs && t0 < end) {
-        spa = bt[uniform(t0 >> 4)];
-        spb = t0 + 16 < end ? bt[uniform((t0 >> 4) + 1)] : -1;
+        spa = bt[uniform(t0 >> bs_shift)];
+        spb = t0 + 16 < end ? bt[uniform((t0 + 16) >> bs_shift)] : -1;
     }
 
     // Q^T fragments: head n (zeros for n >= G), dims 32 s + 8 g .. +7.
@@ -1064,24 +1068,26 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     };
 
     const size_t page_stride = (size_t)hkv * bs * D;  // elements
-    // Whole pairs of 16-token pages: two wave-uniform page ids (loaded one
-    // pair ahead), every K/V load at page base + lane offset.
+    // Whole pairs of 16-token chunks, each in one page (a power of two of at
+    // least 16 tokens): two wave-uniform page ids (loaded one pair ahead),
+    // every K/V load at chunk base + lane offset.
     {
-        const uint32_t kv_off = (uint32_t)(kvh * 16 * D);
-        uint32_t koff[KS], voff[4];  // byte offsets inside a page
+        uint32_t koff[KS], voff[4];  // byte offsets from the first row of a chunk
 #pragma unroll
-        for (int s = 0; s < KS; ++s) koff[s] = (kv_off + n * D + 32 * s + 8 * g) * 2;
+        for (int s = 0; s < KS; ++s) koff[s] = (n * D + 32 * s + 8 * g) * 2;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) voff[r] = (kv_off + (4 * g + r) * D + DPL * n) * 2;
+        for (int r = 0; r < 4; ++r) voff[r] = ((4 * g + r) * D + DPL * n) * 2;
+        const f16 *kch = kc + (size_t)kvh * bs * D, *vch = vc + (size_t)kvh * bs * D;  // this kv head of page 0
+        auto chunk = [&](const f16* cache, int pid, int t) {
+            return reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + (t & (bs - 1)) * D);
+        };
         const bool unused[8] = {};
         while (fast_bs && t0 + T::TOK <= end && (unsigned)spa < (unsigned)num_blocks &&
                (unsigned)spb < (unsigned)num_blocks) {
             f16x8 ka[KS], kb[KS];
             vrow_t va[4], vb[4];
-            const char* kpa = reinterpret_cast<const char*>(kc + (size_t)spa * page_stride);
-            const char* kpb = reinterpret_cast<const char*>(kc + (size_t)spb * page_stride);
-            const char* vpa = reinterpret_cast<const char*>(vc + (size_t)spa * page_stride);
-            const char* vpb = reinterpret_cast<const char*>(vc + (size_t)spb * page_stride);
+            const char *kpa = chunk(kch, spa, t0), *kpb = chunk(kch, spb, t0 + 16);
+            const char *vpa = chunk(vch, spa, t0), *vpb = chunk(vch, spb, t0 + 16);
 #pragma unroll
             for (int s = 0; s < KS; ++s) {  // streamed once: non-temporal
                 ka[s] = __builtin_nontemporal_load(reinterpret_cast<const f16x8*>(kpa + koff[s]));
@@ -1094,8 +1100,8 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
             }
             const int tn = t0 + stride;
             if (tn < end) {  // the next pair's page ids (page B only if it holds a token)
-                spa = bt[uniform(tn >> 4)];
-                spb = tn + 16 < end ? bt[uniform((tn >> 4) + 1)] : -1;
+                spa = bt[uniform(tn >> bs_shift)];
+                spb = tn + 16 < end ? bt[uniform((tn + 16) >> bs_shift)] : -1;
             }
             if (balance) progress_priority(t0 - start, end - start);
             step(ka, kb, va, vb, unused, std::false_type{});
@@ -1113,11 +1119,9 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
             f16x8 ka[KS], kb[KS];
             vrow_t va[4], vb[4];
             bool valid[8];
-            const int pb = hasb ? spb : spa;  // no row of page B is read when it holds no token
-            const char* kpa = reinterpret_cast<const char*>(kc + (size_t)spa * page_stride);
-            const char* vpa = reinterpret_cast<const char*>(vc + (size_t)spa * page_stride);
-            const char* kpb = reinterpret_cast<const char*>(kc + (size_t)pb * page_stride);
-            const char* vpb = reinterpret_cast<const char*>(vc + (size_t)pb * page_stride);
+            const int pb = hasb ? spb : spa;  // no row of chunk B is read when it holds no token
+            const char *kpa = chunk(kch, spa, t0), *kpb = chunk(kch, pb, t0 + 16);
+            const char *vpa = chunk(vch, spa, t0), *vpb = chunk(vch, pb, t0 + 16);
             const bool ka_ok = t0 + n < end, kb_ok = t0 + 16 + n < end;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {

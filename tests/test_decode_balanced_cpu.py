@@ -38,7 +38,11 @@ def cut(lens, workers, cap, gran, ulp=0):
         count = int(n.sum())
         if count <= workers:
             break
-        size = up(size + 1 + int(F(size) * F(count - workers) * rcp(workers, ulp))) if it < 6 else up(cap)
+        if it == 0:
+            more = int(F(c.sum()) * rcp(max(1, workers - len(lens) // 2), ulp))
+        else:
+            more = size + int(F(size) * F(count - workers) * rcp(workers, ulp))
+        size = up(max(size, more) + 1) if it < 6 else up(cap)
     segs = []
     for b, (ctx, ns) in enumerate(zip(c, n)):
         length = up((ctx + ns - 1) // ns)
