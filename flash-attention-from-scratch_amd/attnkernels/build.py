@@ -40,7 +40,7 @@ CPP_SOURCES = ["capi.cpp"]
 # does not know the feature, which is harmless.
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-               "-munsafe-fp-atomics", "-Wall", "-Wno-unused-function"]
+               "-munsafe-fp-atomics", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wall", "-Wno-unused-function"]
 
 
 def ext_path() -> Path:
