@@ -52,7 +52,7 @@ struct DecodeArgs {
     // context lengths they find (each at most token_cap), into at most
     // num_splits splits per kv head, of `partition` tokens or more; counters
     // are set, and the partials are [hq, num_splits] rows.
-    bool balanced = false;
+    bool balanced = false, longest_first = false;
     int64_t token_cap = 0;
     float sl2;             // scale * log2(e)
     void* stream;
@@ -79,8 +79,13 @@ hipError_t decode_launch(const DecodeArgs& a);
 constexpr int64_t kBalancedMaxBatch = 64;
 constexpr int64_t kBalancedMinSplit = 256;
 // Workgroups per kv head of a balanced launch for these sizes (max_ctx: the
-// longest context, cap: the most tokens read of one), 0: use fixed splits.
-int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap);
+// longest context, cap: the most tokens read of one), 0: use fixed splits; and
+// whether its splits run longest first.
+struct BalancedPlan {
+    int64_t workers;
+    bool longest_first;
+};
+BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap);
 
 // Size of the static per-GPU split-partials array behind
 // ak_paged_decode_noalloc, and its device address on the current GPU

@@ -141,16 +141,16 @@ void set_partials(ak::DecodeArgs& a, void* buf, size_t rows) {
     a.l_part = a.m_part + rows;
 }
 
-// Workgroups per kv head of the balanced launch for these sizes; 0: none
-// (invalid sizes, or fixed splits serve).  The most tokens it reads of a
-// sequence are those fixed splits of `partition` tokens would read.
-int64_t balanced_workers(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
-                         int64_t max_context_len, int64_t partition) {
+// The balanced launch for these sizes; no workers: none (invalid sizes, or
+// fixed splits serve).  The most tokens it reads of a sequence are those fixed
+// splits of `partition` tokens would read.
+ak::BalancedPlan balanced_plan(int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                               int64_t max_context_len, int64_t partition) {
     if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 || head_dim <= 0 || partition <= 0 ||
         max_context_len < 1 || max_context_len > INT_MAX - partition)
-        return 0;
+        return {0, false};
     const int64_t cap = (max_context_len + partition - 1) / partition * partition;
-    return ak::decode_balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len, cap);
+    return ak::decode_balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_context_len, cap);
 }
 
 }  // namespace
@@ -255,8 +255,9 @@ int ak_paged_decode_fused(const void* q, const void* k_cache, const void* v_cach
 
 size_t ak_paged_decode_balanced_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads,
                                                int64_t head_dim, int64_t max_context_len, int64_t partition) {
-    return partials_bytes(1, num_heads, balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len,
-                                                         partition), head_dim);
+    const int64_t workers =
+        balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_context_len, partition).workers;
+    return partials_bytes(1, num_heads, workers, head_dim);
 }
 
 int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
@@ -270,7 +271,8 @@ int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_c
                                head_dim, num_blocks, block_size, max_blocks_per_seq, max_context_len, scale,
                                partition, stream, a);
     if (rc != AK_OK || batch == 0) return rc;
-    const int64_t workers = balanced_workers(batch, num_heads, num_kv_heads, head_dim, max_context_len, partition);
+    const auto [workers, longest_first] =
+        balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_context_len, partition);
     if (workers == 0)
         return fail(AK_ERR_UNSUPPORTED, "paged_decode_balanced: fixed splits serve these sizes "
                                         "(ak_paged_decode_balanced_workspace_size is 0)");
@@ -286,6 +288,7 @@ int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_c
         return fail(AK_ERR_INVALID_ARGUMENT, "paged_decode_balanced: workspace must be 16-byte aligned");
     a.token_cap = std::min(a.num_splits * a.partition, a.max_blocks * a.bs);
     a.balanced = true;
+    a.longest_first = longest_first;
     a.partition = ak::kBalancedMinSplit;
     a.num_splits = workers;
     a.counters = counters;

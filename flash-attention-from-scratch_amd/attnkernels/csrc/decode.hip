@@ -169,6 +169,23 @@ __device__ __forceinline__ int wave_scan(int x) {
     return x;
 }
 
+// Maximum over the lanes of a wave of values >= 0.
+__device__ __forceinline__ float wave_max(float x) {
+    auto shifted = [](float v, auto ctrl, auto rows) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                     decltype(ctrl)::value, decltype(rows)::value,
+                                                                     0xF, true));
+    };
+    using std::integral_constant;
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{}));
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{}));
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{}));
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{}));
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}));
+    x = fmaxf(x, shifted(x, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{}));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+}
+
 // Splits of about equal size, cut from the context lengths the kernel finds:
 // grid (kv head, workgroup), `workers` workgroups per kv head, one split each.
 // A fixed partition gives a ragged batch workgroups of very different
@@ -178,9 +195,12 @@ __device__ __forceinline__ int wave_scan(int x) {
 // multiple of GRAN, the tokens of one workgroup iteration) for which the
 // sequences have at most `workers` splits in all, and cuts each sequence into
 // that many even ones.  Every workgroup of every kv head finds the same cut.
+// longest_first: the splits run in the order of their lengths, in four classes
+// by the quarters of the longest, so that a launch of more workgroups than
+// the GPU holds does not end on a long one.
 template <int G, int GRAN>
 __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_lens, int kvh, int min_split,
-                                                    int workers, int batch, int cap, int lane) {
+                                                    int workers, int batch, int cap, int longest_first, int lane) {
     const int c = lane < batch ? min(max(ctx_lens[lane], 0), cap) : -1;
     const int total = __builtin_amdgcn_readlane(wave_scan(max(c, 0)), 63);
     auto round_up = [](int x) { return (x + GRAN - 1) / GRAN * GRAN; };
@@ -209,11 +229,26 @@ __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_
     sg.split = sg.ns = sg.start = sg.end = 0;
     sg.slot0 = 0;
     sg.hstride = workers;
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(j >= incl - n && j < incl);
+    int first = incl - n;  // this lane's first workgroup
+    if (longest_first) {
+        const float len = c < 0 ? 0.f : (float)c * __builtin_amdgcn_rcpf((float)n);
+        const float top = wave_max(len);
+        const int quarter = min(3, (int)(4.f * len * __builtin_amdgcn_rcpf(fmaxf(top, 1.f))));
+        if (__builtin_amdgcn_ballot_w64(c >= 0 && quarter < 3)) {
+            int before = 0;
+#pragma unroll
+            for (int k = 3; k >= 0; --k) {
+                const int nk = quarter == k ? n : 0, sum = wave_scan(nk);
+                first = quarter == k ? before + sum - nk : first;
+                before += __builtin_amdgcn_readlane(sum, 63);
+            }
+        }
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(j >= first && j < first + n);
     if (hit) {
         const int l = (int)__builtin_ctzll(hit);
         const int ctx = __builtin_amdgcn_readlane(c, l), ns = __builtin_amdgcn_readlane(n, l);
-        const int base = __builtin_amdgcn_readlane(incl, l) - ns;
+        const int base = __builtin_amdgcn_readlane(first, l);
         // Even splits of a multiple of GRAN tokens.  Each holds a token: len <=
         // size because size is such a multiple, and (ns - 1) * size < ctx.
         const int len = round_up((int)(((unsigned)ctx + ns - 1) / (unsigned)ns));
@@ -328,7 +363,7 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
                     f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                     float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs, int bs_shift,
                     int max_blocks, int num_blocks, int partition, int num_splits, float sl2, int batch,
-                    int cap) {
+                    int cap, int longest_first) {
     using T = DecodeTile<D>;
     constexpr int G = 1;
     __shared__ float red_acc[T::NW][G][D];
@@ -341,7 +376,8 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;  // never index past the table row
-    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                                      longest_first, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -603,7 +639,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
                         f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                         float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                         int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits, float sl2,
-                        int balance, int batch, int cap) {
+                        int balance, int batch, int cap, int longest_first) {
     using T = GqaTile<D, G, NW>;
     constexpr int U = T::U, N = T::N, S = T::S, LB = T::LB;
     // P = 2^(s - m + kPShift): the largest P the fast path accepts is 2^kPMax.
@@ -616,7 +652,8 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;
-    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                                      longest_first, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -941,7 +978,7 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
                              f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                              float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                              int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits,
-                             float sl2, int balance, int batch, int cap) {
+                             float sl2, int balance, int batch, int cap, int longest_first) {
     using T = GqaMfmaTile<D, G, NW>;
     constexpr int KS = T::KS, DPL = T::DPL;
     typedef _Float16 vrow_t __attribute__((ext_vector_type(DPL)));
@@ -955,7 +992,8 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int max_tok = max_blocks * bs;
-    const Segment sg = BALANCED ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                                   longest_first, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -1289,7 +1327,7 @@ static bool one_round(int threads, int64_t wgs) {
     return per_cu > 0 && wgs <= (int64_t)per_cu * cus;
 }
 
-// Balanced splits: the workgroups per kv head, or 0 where fixed splits serve.
+// Balanced splits: the workgroups per kv head (0: fixed splits serve), and their order.
 //   * One sequence has nothing to balance; up to 1024 tokens, or 64 MB of K and
 //     V if all were the longest, the fixed splits leave each workgroup a few
 //     iterations, and finding the cut costs up to 0.5 us more than it gives (8 x
@@ -1306,18 +1344,24 @@ static bool one_round(int threads, int64_t wgs) {
 //     for one head at D = 128, whose four waves of 16 loads gain less from a
 //     cut than a partial second round costs (16 x 100-1200 tokens, Hkv=32: 39.0
 //     us in 512 workgroups, 43.8 in up to 1024).  Where that leaves less than
-//     an eighth, the fixed splits' cheaper start wins (64 of 1-4096, Hkv=32:
-//     367.3 us against 368.3).
+//     an eighth in a single round, there is nothing to balance and the fixed
+//     splits start sooner.
+//   * Past one round the longest splits run first, in four classes (a rank of
+//     each by comparisons with all others costs 2-5 us at 64 sequences, the
+//     classes 0.3): 64 of 1-4096 tokens, Hkv=32 368.9 -> 346.2, 32 of 100-8192
+//     429.8 -> 379.0; 64 of 1-8192, Hq=64, Hkv=8 211.1 -> 197.5; 48 of 100-2000,
+//     Hkv=32, D=64 82.5 -> 76.4.  Equal lengths keep their order: 64 x 2048,
+//     Hkv=32 328.3 -> 329.0.
 // Measured against fixed splits of decode_partition (us a call, back to back;
 // Hq=32, Hkv=8, D=128 unless noted): 16 x 8192 88.9 -> 83.6; 16 ragged 512-8192
 // 65.4 -> 54.6, with Hq=64 77.6 -> 60.9; 32 ragged 64-4096 62.9 -> 55.4; 8 of
 // 500-32000, Hq=16 118.8 -> 103.5; 10 x 22420, D=64 82.9 -> 74.4; 8 x 32768,
 // Hkv=32 678 -> 652 (D=64: 366 -> 331).  768, 1024, 2048 and 4096 workgroups
 // where these rules take 256 or 512 were 1-30% slower.
-int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
+BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
     if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24) ||
         batch * hkv * max_ctx * d * 4 < (int64_t(64) << 20))
-        return 0;
+        return {0, false};
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -1326,7 +1370,9 @@ int64_t decode_balanced_workers(int64_t batch, int64_t hq, int64_t hkv, int64_t 
     const int64_t round = one_head ? 2 * cus : cus;
     const int64_t need = batch + (max_ctx > 8192 ? batch / 2 : one_head ? 0 : (batch + 7) / 8);
     const int64_t workers = (need * hkv + round - 1) / round * round / hkv;
-    return workers * 8 < batch * 9 ? 0 : workers;  // next to no room to cut anything: fixed splits
+    const bool one_round = batch * hkv <= round;
+    if (one_round && workers * 8 < batch * 9) return {0, false};
+    return {workers, !one_round};
 }
 
 template <int D, int G>
@@ -1345,8 +1391,9 @@ static hipError_t launch_decode(const DecodeArgs& a) {
                            (const f16*)a.v_cache, a.block_tables, a.context_lens, (f16*)a.out, a.o_part, a.m_part,
                            a.l_part, counters, (int)a.hkv, (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks,
                            (int)a.partition, (int)a.num_splits, a.sl2, more..., (int)a.batch,
-                           (int)a.token_cap);
+                           (int)a.token_cap, (int)a.longest_first);
     };
+
     auto launch_mode = [&](auto mode) {
         constexpr bool BALANCED = decltype(mode)::value;
         if constexpr (G == 1) {

@@ -42,6 +42,20 @@ def test_matches_oracle(name, g, hkv, d, bs):
     assert max_err(ak.paged_decode(*dev, LONGEST), oracle.paged_decode_fp32(q, kc, vc, bt, short)) < TOL[d]
 
 
+@pytest.mark.parametrize("g,hkv,d", [(1, 16, 128), (1, 8, 64), (2, 8, 128), (8, 8, 64)])
+def test_longest_first(g, hkv, d):
+    """More workgroups than one round, lengths in all four classes, at their edges and empty."""
+    lens = [0, 1, 4096, 1024, 1023, 1025, 2048, 2049, 3072, 3071] + [1 + 37 * i * i % 4096 for i in range(38)]
+    kc, vc, bt, cl = oracle.make_paged_cache([max(1, n) for n in lens], hkv, d, block_size=16, extra_blocks=3, seed=d)
+    cl[0] = 0
+    q = np.random.default_rng(g + d).standard_normal((len(lens), g * hkv, d), dtype=np.float32).astype(np.float16)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, bt, cl)]
+    ref = np.zeros(q.shape, np.float32)
+    ref[1:] = oracle.paged_decode_fp32(q[1:], kc, vc, bt[1:], cl[1:])
+    for _ in range(2):
+        assert max_err(ak.paged_decode(*dev, 8192), ref) < TOL[d]
+
+
 def test_tokens_past_the_longest_context_given_are_cut_as_with_fixed_splits():
     """A length above max_context_len (outside the contract) reads up to the end of the last fixed split."""
     kc, vc, bt, cl = oracle.make_paged_cache([20000, 300], 4, 128, block_size=16, extra_blocks=1, seed=1)

@@ -1,6 +1,6 @@
 """The cut of a batch's contexts into splits that the decode kernels make when
 no partition is given (balanced_segment in decode.hip), replayed lane by lane in
-float32 and int32, and the rule that picks that path (decode_balanced_workers).
+float32 and int32, and the rule that picks that path (decode_balanced_plan).
 
 Every split must hold a token, the splits of a sequence must tile its context,
 and no kv head may need more splits than the launch has workgroups: a split
@@ -77,6 +77,25 @@ def test_every_token_is_in_one_split(gran, ulp):
             assert [at[b] for b in range(len(lens))] == lens, (lens, workers)
 
 
+@pytest.mark.parametrize("ulp", [-1, 0, 1])
+def test_longest_first_order_is_a_permutation(ulp):
+    """The workgroups of the sequences, in classes by the quarters of the longest split: no gap, no overlap."""
+    for lens in batches():
+        c, n = np.asarray(lens, np.int64), None
+        segs, count, _ = cut(lens, 2 * len(lens), -(-max(lens) // 256) * 256, 128, ulp)
+        n = np.array([sum(1 for s in segs if s[0] == b) for b in range(len(lens))])
+        length = c.astype(F) * np.array([rcp(x, ulp) for x in n])
+        quarter = np.minimum(3, (F(4) * length * rcp(max(length.max(), F(1)), ulp)).astype(np.int64))
+        first, before = np.zeros(len(lens), np.int64), 0
+        for k in (3, 2, 1, 0):
+            nk = np.where(quarter == k, n, 0)
+            first = np.where(quarter == k, before + nk.cumsum() - nk, first)
+            before += nk.sum()
+        assert sorted(int(f) + i for f, m in zip(first, n) for i in range(m)) == list(range(count))
+        assert all(length[a] >= length[b] or quarter[a] == quarter[b]
+                   for a in range(len(lens)) for b in range(len(lens)) if first[a] < first[b])
+
+
 def test_even_batches_are_cut_evenly():
     for batch, workers, ctx in ((16, 32, 8192), (8, 32, 8192), (4, 64, 30000), (10, 32, 22420)):
         segs, _, _ = cut([ctx] * batch, workers, ctx + 255, 128)
@@ -124,8 +143,8 @@ def test_rule(lib):
                     if batch * hkv * ctx * d * 4 < 64 << 20:
                         assert w == 0
                         continue
-                    if w == 0:  # no room to cut: about one workgroup per sequence
-                        assert hq == hkv and d == 128 and ctx <= 8192
+                    if w == 0:  # no room to cut in one round: about one workgroup per sequence
+                        assert hq == hkv and d == 128 and ctx <= 8192 and batch * hkv <= 512
                         continue
                     assert w >= batch + (batch // 2 if ctx > 8192 else 0) and w <= 65535
                     unit = 512 if hq == hkv and d == 128 else 256
