@@ -52,7 +52,8 @@ struct DecodeArgs {
     // context lengths they find (each at most token_cap), into at most
     // num_splits splits per kv head, of `partition` tokens or more; counters
     // are set, and the partials are [hq, num_splits] rows.
-    bool balanced = false, longest_first = false;
+    bool balanced = false;
+    int order = 0;         // of balanced splits: kLongestFirst, kEqualUncut
     int64_t token_cap = 0;
     float sl2;             // scale * log2(e)
     void* stream;
@@ -80,10 +81,11 @@ constexpr int64_t kBalancedMaxBatch = 64;
 constexpr int64_t kBalancedMinSplit = 256;
 // Workgroups per kv head of a balanced launch for these sizes (max_ctx: the
 // longest context, cap: the most tokens read of one), 0: use fixed splits; and
-// whether its splits run longest first.
+// the flags of their order.
+constexpr int kLongestFirst = 1, kEqualUncut = 2;
 struct BalancedPlan {
     int64_t workers;
-    bool longest_first;
+    int order;
 };
 BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap);
 

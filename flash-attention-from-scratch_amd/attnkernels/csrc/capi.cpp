@@ -148,7 +148,7 @@ ak::BalancedPlan balanced_plan(int64_t batch, int64_t num_heads, int64_t num_kv_
                                int64_t max_context_len, int64_t partition) {
     if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0 || head_dim <= 0 || partition <= 0 ||
         max_context_len < 1 || max_context_len > INT_MAX - partition)
-        return {0, false};
+        return {0, 0};
     const int64_t cap = (max_context_len + partition - 1) / partition * partition;
     return ak::decode_balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_context_len, cap);
 }
@@ -271,7 +271,7 @@ int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_c
                                head_dim, num_blocks, block_size, max_blocks_per_seq, max_context_len, scale,
                                partition, stream, a);
     if (rc != AK_OK || batch == 0) return rc;
-    const auto [workers, longest_first] =
+    const auto [workers, order] =
         balanced_plan(batch, num_heads, num_kv_heads, head_dim, max_context_len, partition);
     if (workers == 0)
         return fail(AK_ERR_UNSUPPORTED, "paged_decode_balanced: fixed splits serve these sizes "
@@ -288,7 +288,7 @@ int ak_paged_decode_balanced(const void* q, const void* k_cache, const void* v_c
         return fail(AK_ERR_INVALID_ARGUMENT, "paged_decode_balanced: workspace must be 16-byte aligned");
     a.token_cap = std::min(a.num_splits * a.partition, a.max_blocks * a.bs);
     a.balanced = true;
-    a.longest_first = longest_first;
+    a.order = order;
     a.partition = ak::kBalancedMinSplit;
     a.num_splits = workers;
     a.counters = counters;

@@ -27,6 +27,7 @@
 //     out as the MFMA operands (see there);
 //   * the lane groups of a wave and the waves of a workgroup are merged once,
 //     at the end, by the same LSE rule.
+#include <algorithm>
 #include "attn_kernels.hpp"
 #include "wave.hpp"
 
@@ -186,26 +187,38 @@ __device__ __forceinline__ float wave_max(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
 }
 
+// The cut of the dot-product kernels is a multiple of this, that of the matrix
+// kernel of its 32-token wave chunk, not of a whole iteration of all waves
+// (128 or 256 tokens): 16 ragged 512-8192 tokens, D = 128, Hkv=8, Hq=64 60.4 ->
+// 57.3 us, Hq=32 53.8 -> 53.0; 32 for the dot-product kernels is no better
+// (16 of 2000-20000, G = 4: 71.7 -> 72.0).
+constexpr int kDotGran = 64;
+
 // Splits of about equal size, cut from the context lengths the kernel finds:
 // grid (kv head, workgroup), `workers` workgroups per kv head, one split each.
 // A fixed partition gives a ragged batch workgroups of very different
 // lengths, and most of the grid may be empty; HBM then idles while the longest
 // ones finish.  Here every wave reads all the lengths (one load, a lane per
 // sequence), looks for the smallest split size (at least min_split tokens, a
-// multiple of GRAN, the tokens of one workgroup iteration) for which the
-// sequences have at most `workers` splits in all, and cuts each sequence into
-// that many even ones.  Every workgroup of every kv head finds the same cut.
-// longest_first: the splits run in the order of their lengths, in four classes
-// by the quarters of the longest, so that a launch of more workgroups than
-// the GPU holds does not end on a long one.
+// multiple of GRAN) for which the sequences have at most `workers` splits in
+// all, and cuts each sequence into that many even ones.  Every workgroup of
+// every kv head finds the same cut.  `order` holds flags:
+//   kLongestFirst: the splits run in the order of their lengths, in four
+//     classes by the quarters of the longest, so that a launch of more
+//     workgroups than the GPU holds does not end on a long one.
+//   kEqualUncut: sequences within an eighth of the longest stay whole.
 template <int G, int GRAN>
 __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_lens, int kvh, int min_split,
-                                                    int workers, int batch, int cap, int longest_first, int lane) {
+                                                    int workers, int batch, int cap, int order, int lane) {
     const int c = lane < batch ? min(max(ctx_lens[lane], 0), cap) : -1;
     const int total = __builtin_amdgcn_readlane(wave_scan(max(c, 0)), 63);
     auto round_up = [](int x) { return (x + GRAN - 1) / GRAN * GRAN; };
     // No smaller size can do; even batches take this one.
     int size = max(min_split, round_up(1 + (int)((float)(total - 1) * __builtin_amdgcn_rcpf((float)workers))));
+    if (order & kEqualUncut) {
+        const int longest = (int)wave_max((float)max(c, 0));
+        if (!__builtin_amdgcn_ballot_w64(c >= 0 && c * 8 < longest * 7)) size = max(size, round_up(longest));
+    }
     int n, incl;
     for (int it = 0;; ++it) {
         // ceil(c / size), a float quotient put right by one step either way
@@ -230,7 +243,7 @@ __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_
     sg.slot0 = 0;
     sg.hstride = workers;
     int first = incl - n;  // this lane's first workgroup
-    if (longest_first) {
+    if (order & kLongestFirst) {
         const float len = c < 0 ? 0.f : (float)c * __builtin_amdgcn_rcpf((float)n);
         const float top = wave_max(len);
         const int quarter = min(3, (int)(4.f * len * __builtin_amdgcn_rcpf(fmaxf(top, 1.f))));
@@ -363,7 +376,7 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
                     f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                     float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs, int bs_shift,
                     int max_blocks, int num_blocks, int partition, int num_splits, float sl2, int batch,
-                    int cap, int longest_first) {
+                    int cap, int order) {
     using T = DecodeTile<D>;
     constexpr int G = 1;
     __shared__ float red_acc[T::NW][G][D];
@@ -376,8 +389,8 @@ paged_decode_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, const
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;  // never index past the table row
-    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
-                                                                      longest_first, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, kDotGran>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                               order, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -639,7 +652,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
                         f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                         float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                         int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits, float sl2,
-                        int balance, int batch, int cap, int longest_first) {
+                        int balance, int batch, int cap, int order) {
     using T = GqaTile<D, G, NW>;
     constexpr int U = T::U, N = T::N, S = T::S, LB = T::LB;
     // P = 2^(s - m + kPShift): the largest P the fast path accepts is 2^kPMax.
@@ -652,8 +665,8 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int gi = lane / T::LPT, li = lane % T::LPT;
     const int max_tok = max_blocks * bs;
-    const Segment sg = BALANCED ? balanced_segment<G, T::NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
-                                                                      longest_first, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, kDotGran>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                               order, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -978,7 +991,7 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
                              f16* __restrict__ out, float* __restrict__ o_part, float* __restrict__ m_part,
                              float* __restrict__ l_part, int32_t* __restrict__ counters, int hkv, int bs,
                              int bs_shift, int max_blocks, int num_blocks, int partition, int num_splits,
-                             float sl2, int balance, int batch, int cap, int longest_first) {
+                             float sl2, int balance, int batch, int cap, int order) {
     using T = GqaMfmaTile<D, G, NW>;
     constexpr int KS = T::KS, DPL = T::DPL;
     typedef _Float16 vrow_t __attribute__((ext_vector_type(DPL)));
@@ -992,8 +1005,8 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int max_tok = max_blocks * bs;
-    const Segment sg = BALANCED ? balanced_segment<G, NW * T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
-                                                                   longest_first, lane)
+    const Segment sg = BALANCED ? balanced_segment<G, T::TOK>(ctx_lens, kvh, partition, num_splits, batch, cap,
+                                                              order, lane)
                                 : fixed_segment(ctx_lens, kvh * G, hq, max_tok, partition, num_splits);
     const int b = sg.b, split = sg.split, start = sg.start, end = sg.end;
     if (BALANCED && b < 0) return;
@@ -1336,43 +1349,73 @@ static bool one_round(int threads, int64_t wgs) {
 //     31.1 fixed, 23.3 balanced).
 //   * More than 64 sequences do not fit one load of lengths by a wave; a batch
 //     that large fills the GPU by itself.
-//   * Workgroups in whole rounds of the GPU: one 8-wave workgroup per CU
-//     (grouped-query kernels), two 4-wave ones (one head, D = 128), or as many
-//     rounds of those as give every sequence a workgroup and leave some to cut
-//     the longer ones: an eighth of the batch, half of it past 8192 tokens (one
-//     long sequence among short ones; the fixed rule splits there too), none
-//     for one head at D = 128, whose four waves of 16 loads gain less from a
-//     cut than a partial second round costs (16 x 100-1200 tokens, Hkv=32: 39.0
-//     us in 512 workgroups, 43.8 in up to 1024).  Where that leaves less than
-//     an eighth in a single round, there is nothing to balance and the fixed
+//   * Workgroups in whole rounds of the GPU (one 8-wave workgroup per CU, two
+//     or more of 4 waves), because HBM idles in a partial one: 384 workgroups
+//     measure 10-25% behind 256 and 512.
+//   * 1.7 of them per sequence where the batch itself is up to 512: with fewer
+//     the longest sequences cannot be cut (24 of 512-8192 tokens, Hkv=8, in 256
+//     and 512 or 768 workgroups: Hq=64 90.1, 80; Hq=16 80.0, 74; D=64, Hq=32
+//     47.1, 41; 56 of them, Hq=64, in 512 and 768: 188, 170); with more each
+//     split starts and merges for less (16 of them, Hq=32: 52.9 in 256, 54.8 in
+//     512, 57.5 in 1024).
+//     Past 512, 1.1 of them (1.5 for contexts past 8192: one long sequence
+//     among short ones): the order below does the balancing.
+//   * Up to 1024 workgroups, the first size of which equal sequences, each cut
+//     alike, fill more than three quarters (24 x 4096, Hq=32: 68.2 in 512, 67.0
+//     in 768).  Eight heads at D = 128 start at 512: the matrix-core kernel's 8
+//     waves are further apart than two workgroups of 4 (12 x 4096 41.4 in 256,
+//     37.8 in 512; 16 of 512-8192 63.3, 56.1).
+//   * One head at D = 128 takes as many rounds of 512 as give every sequence a
+//     workgroup (1.5 past 8192 tokens): four waves of 16 loads gain less from a
+//     cut than a second round costs (16 x 100-1200 tokens, Hkv=32: 39.0 us in
+//     512 workgroups, 43.8 in up to 1024).  Where that leaves less than an
+//     eighth in a single round, there is nothing to balance and the fixed
 //     splits start sooner.
-//   * Past one round the longest splits run first, in four classes (a rank of
-//     each by comparisons with all others costs 2-5 us at 64 sequences, the
+//   * Past 512 workgroups the longest splits run first, in four classes (a rank
+//     of each by comparisons with all others costs 2-5 us at 64 sequences, the
 //     classes 0.3): 64 of 1-4096 tokens, Hkv=32 368.9 -> 346.2, 32 of 100-8192
-//     429.8 -> 379.0; 64 of 1-8192, Hq=64, Hkv=8 211.1 -> 197.5; 48 of 100-2000,
-//     Hkv=32, D=64 82.5 -> 76.4.  Equal lengths keep their order: 64 x 2048,
-//     Hkv=32 328.3 -> 329.0.
+//     429.8 -> 379.0; 56 of 512-8192, Hq=64, Hkv=8 193.3 -> 169.9.
+//   * Sequences of about one length stay whole where the batch fills two rounds
+//     or more: 64 x 4096, Hkv=8: Hq=32 169.9 -> 164.0, Hq=64 176.0 -> 163.7
+//     (fixed splits 163.6 and 161.6).
 // Measured against fixed splits of decode_partition (us a call, back to back;
-// Hq=32, Hkv=8, D=128 unless noted): 16 x 8192 88.9 -> 83.6; 16 ragged 512-8192
-// 65.4 -> 54.6, with Hq=64 77.6 -> 60.9; 32 ragged 64-4096 62.9 -> 55.4; 8 of
-// 500-32000, Hq=16 118.8 -> 103.5; 10 x 22420, D=64 82.9 -> 74.4; 8 x 32768,
-// Hkv=32 678 -> 652 (D=64: 366 -> 331).  768, 1024, 2048 and 4096 workgroups
-// where these rules take 256 or 512 were 1-30% slower.
+// Hq=32, Hkv=8, D=128 unless noted): 16 x 8192 89.3 -> 84.4; 16 ragged 512-8192
+// 63.4 -> 52.9, with Hq=64 76.8 -> 57.3; 24 of them 103.4 -> 92.8, 40 127.7 ->
+// 118.7; 64 of 1-8192 197.8 -> 182.0, with Hq=64 235.7 -> 193.7; 8 of 500-32000,
+// Hq=16 114.1 -> 98.0; 8 x 32768, Hkv=32 678 -> 652 (D=64: 366 -> 331).
+// Behind them: 22 x 4096 62.3 -> 63.0, 33 x 4096 98.2 -> 100.9, 24 x 4096, Hq=64
+// 70.6 -> 72.0, 64 x 2048, Hq=64 82.0 -> 84.5.
 BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
     if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24) ||
         batch * hkv * max_ctx * d * 4 < (int64_t(64) << 20))
-        return {0, false};
+        return {0, 0};
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const bool one_head = hq == hkv && d == 128;
     const int64_t round = one_head ? 2 * cus : cus;
-    const int64_t need = batch + (max_ctx > 8192 ? batch / 2 : one_head ? 0 : (batch + 7) / 8);
-    const int64_t workers = (need * hkv + round - 1) / round * round / hkv;
-    const bool one_round = batch * hkv <= round;
-    if (one_round && workers * 8 < batch * 9) return {0, false};
-    return {workers, !one_round};
+    int64_t k, workers;
+    if (one_head) {
+        const int64_t need = batch + (max_ctx > 8192 ? batch / 2 : 0);
+        k = (need * hkv + round - 1) / round;
+        workers = k * round / hkv;
+    } else {
+        const bool cut = batch * hkv <= 2 * cus;
+        k = (batch * hkv * (cut ? 17 : max_ctx > 8192 ? 15 : 11) + 10 * cus - 1) / (10 * cus);
+        if (cut && hq == 8 * hkv && d == 128) k = std::max<int64_t>(k, 2);
+        for (int64_t i = k; cut && i <= std::max<int64_t>(k, 4); ++i) {
+            const int64_t w = i * round / hkv;
+            if (w / batch * batch * 4 > w * 3) {
+                k = i;
+                break;
+            }
+        }
+        workers = k * round / hkv;
+    }
+    if (batch * hkv <= round && workers * 8 < batch * 9) return {0, 0};
+    const bool rounds = !one_head && batch * hkv >= 2 * cus && batch * hkv % cus == 0;
+    return {workers, (workers * hkv > 2 * cus ? kLongestFirst : 0) | (rounds ? kEqualUncut : 0)};
 }
 
 template <int D, int G>
@@ -1391,7 +1434,7 @@ static hipError_t launch_decode(const DecodeArgs& a) {
                            (const f16*)a.v_cache, a.block_tables, a.context_lens, (f16*)a.out, a.o_part, a.m_part,
                            a.l_part, counters, (int)a.hkv, (int)a.bs, bs_shift, (int)a.max_blocks, (int)a.num_blocks,
                            (int)a.partition, (int)a.num_splits, a.sl2, more..., (int)a.batch,
-                           (int)a.token_cap, (int)a.longest_first);
+                           (int)a.token_cap, (int)a.order);
     };
 
     auto launch_mode = [&](auto mode) {

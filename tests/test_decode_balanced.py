@@ -56,6 +56,18 @@ def test_longest_first(g, hkv, d):
         assert max_err(ak.paged_decode(*dev, 8192), ref) < TOL[d]
 
 
+@pytest.mark.parametrize("g,d", [(4, 128), (8, 128), (2, 64)])
+@pytest.mark.parametrize("shortest", [1792, 1791])  # within an eighth of the longest: whole; a token less: cut
+def test_about_equal_sequences(g, d, shortest):
+    lens = [2048, shortest] + [1800 + 13 * i % 249 for i in range(62)]
+    kc, vc, bt, cl = oracle.make_paged_cache(lens, 8, d, block_size=16, extra_blocks=3, seed=d)
+    q = np.random.default_rng(g + d).standard_normal((len(lens), g * 8, d), dtype=np.float32).astype(np.float16)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, kc, vc, bt, cl)]
+    ref = oracle.paged_decode_fp32(q, kc, vc, bt, cl)
+    for _ in range(2):
+        assert max_err(ak.paged_decode(*dev, 2048), ref) < TOL[d]
+
+
 def test_tokens_past_the_longest_context_given_are_cut_as_with_fixed_splits():
     """A length above max_context_len (outside the contract) reads up to the end of the last fixed split."""
     kc, vc, bt, cl = oracle.make_paged_cache([20000, 300], 4, 128, block_size=16, extra_blocks=1, seed=1)
