@@ -23,7 +23,7 @@ LONGEST = 1 << 16  # max_context_len given, so that even the small batches are c
 
 @pytest.mark.parametrize("name", BATCHES)
 @pytest.mark.parametrize("g,hkv,d,bs", [(1, 4, 128, 16), (1, 2, 64, 8), (2, 2, 128, 16), (4, 8, 128, 16),
-                                        (4, 2, 64, 32), (8, 4, 128, 16), (8, 2, 64, 12)])
+                                        (4, 2, 64, 32), (8, 4, 128, 16), (8, 2, 64, 12), (8, 2, 128, 64), (4, 2, 128, 256)])
 def test_matches_oracle(name, g, hkv, d, bs):
     lens = BATCHES[name]
     kc, vc, bt, cl = oracle.make_paged_cache([max(1, n) for n in lens], hkv, d, block_size=bs, extra_blocks=3, seed=g)
