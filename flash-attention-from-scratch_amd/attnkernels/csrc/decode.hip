@@ -1364,7 +1364,10 @@ static bool one_round(int threads, int64_t wgs) {
 //     alike, fill more than three quarters (24 x 4096, Hq=32: 68.2 in 512, 67.0
 //     in 768).  Eight heads at D = 128 start at 512: the matrix-core kernel's 8
 //     waves are further apart than two workgroups of 4 (12 x 4096 41.4 in 256,
-//     37.8 in 512; 16 of 512-8192 63.3, 56.1).
+//     37.8 in 512; 16 of 512-8192 63.3, 56.1), but not below 96 of sequences
+//     times kv heads, where the merges cost more (4 x 8192: 26.3, 28.7).
+//   * More than 32 workgroups per sequence are too many for the merge in the
+//     decode kernel: fixed splits (2 x 100000, Hkv=1, G = 8: 28.2 us, 60.7 cut).
 //   * One head at D = 128 takes as many rounds of 512 as give every sequence a
 //     workgroup (1.5 past 8192 tokens): four waves of 16 loads gain less from a
 //     cut than a second round costs (16 x 100-1200 tokens, Hkv=32: 39.0 us in
@@ -1403,7 +1406,7 @@ BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_
     } else {
         const bool cut = batch * hkv <= 2 * cus;
         k = (batch * hkv * (cut ? 17 : max_ctx > 8192 ? 15 : 11) + 10 * cus - 1) / (10 * cus);
-        if (cut && hq == 8 * hkv && d == 128) k = std::max<int64_t>(k, 2);
+        if (cut && hq == 8 * hkv && d == 128 && batch * hkv * 8 >= 3 * cus) k = std::max<int64_t>(k, 2);
         for (int64_t i = k; cut && i <= std::max<int64_t>(k, 4); ++i) {
             const int64_t w = i * round / hkv;
             if (w / batch * batch * 4 > w * 3) {
@@ -1414,6 +1417,7 @@ BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_
         workers = k * round / hkv;
     }
     if (batch * hkv <= round && workers * 8 < batch * 9) return {0, 0};
+    if (workers > kFusedMaxSplits * batch) return {0, 0};
     const bool rounds = !one_head && batch * hkv >= 2 * cus && batch * hkv % cus == 0;
     return {workers, (workers * hkv > 2 * cus ? kLongestFirst : 0) | (rounds ? kEqualUncut : 0)};
 }

@@ -143,12 +143,17 @@ def test_rule(lib):
                     if batch * hkv * ctx * d * 4 < 64 << 20:
                         assert w == 0
                         continue
+                    if batch * 32 * hkv < (512 if hq == hkv and d == 128 else 256):  # more splits than the decode kernel merges
+                        assert w == 0
+                        continue
                     if w == 0:  # no room to cut in one round: about one workgroup per sequence
                         assert hq == hkv and d == 128 and ctx <= 8192 and batch * hkv <= 512
                         continue
                     assert w >= batch + (batch // 2 if ctx > 8192 else 0) and w <= 65535
                     unit = 512 if hq == hkv and d == 128 else 256
                     assert w * hkv % unit > unit - hkv or w * hkv % unit == 0
+    assert workers(lib, 2, 8, 1, 128, 100000) == 0 and workers(lib, 8, 8, 1, 128, 100000) == 256
+    assert workers(lib, 8, 64, 8, 128, 8192) == 32 and workers(lib, 12, 64, 8, 128, 8192) == 64
     assert workers(lib, 16, 32, 8, 128, 8192) == 32 and workers(lib, 16, 32, 32, 128, 8192) == 0 and workers(lib, 8, 32, 32, 128, 8192) == 16
 
 
