@@ -144,7 +144,9 @@ int ak_paged_decode_fused(const void *q, const void *k_cache, const void *v_cach
  * attnkernels/csrc/paged_decode.cu:73-77).  The size function returns the bytes
  * of the workspace on the current device, or 0 for sizes that fixed splits
  * serve (one sequence, more than 64, max_context_len up to 1024, less than 64
- * MB of K and V at max_context_len, invalid sizes): the call is then refused with AK_ERR_UNSUPPORTED.  `partition` only
+ * MB of K and V at max_context_len, so few sequences and kv heads that each
+ * would get more than 32 splits, invalid sizes): the call is then refused with
+ * AK_ERR_UNSUPPORTED.  `partition` only
  * bounds the tokens read of a sequence, as in ak_paged_decode: those below the
  * smallest multiple of it >= max_context_len.  counters is required.  Arguments,
  * results and errors are otherwise those of ak_paged_decode_fused. */
