@@ -29,6 +29,7 @@
 //     at the end, by the same LSE rule.
 #include <algorithm>
 #include "attn_kernels.hpp"
+#include "index_math.hpp"
 #include "wave.hpp"
 
 #include <type_traits>
@@ -841,7 +842,7 @@ paged_decode_gqa_kernel(const f16* __restrict__ q, const f16* __restrict__ kc, c
     int t0 = start + w * T::TOK;
     {
         auto load_kv = [&](const f16* cache, int pid, int t, f16x8 (&r)[U]) {
-            const char* base = reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + (t & (bs - 1)) * D);
+            const char* base = reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + page_row_offset(t, bs, D));
 #pragma unroll
             for (int u = 0; u < U; ++u)  // streamed once: non-temporal
                 r[u] = __builtin_nontemporal_load(reinterpret_cast<const f16x8*>(base + lane_off[u]));
@@ -1130,7 +1131,7 @@ paged_decode_gqa_mfma_kernel(const f16* __restrict__ q, const f16* __restrict__ 
         for (int r = 0; r < 4; ++r) voff[r] = ((4 * g + r) * D + DPL * n) * 2;
         const f16 *kch = kc + (size_t)kvh * bs * D, *vch = vc + (size_t)kvh * bs * D;  // this kv head of page 0
         auto chunk = [&](const f16* cache, int pid, int t) {
-            return reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + (t & (bs - 1)) * D);
+            return reinterpret_cast<const char*>(cache + (size_t)pid * page_stride + page_row_offset(t, bs, D));
         };
         const bool unused[8] = {};
         while (fast_bs && t0 + T::TOK <= end && (unsigned)spa < (unsigned)num_blocks &&
