@@ -222,12 +222,8 @@ __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_
     }
     int n, incl;
     for (int it = 0;; ++it) {
-        // ceil(c / size), a float quotient put right by one step either way
-        // (c < 2^24), at least 1 (an empty sequence's workgroup writes its zero rows).
-        n = (int)((float)c * __builtin_amdgcn_rcpf((float)size));
-        n += n * size < c ? 1 : 0;
-        n -= (n - 1) * size >= c ? 1 : 0;
-        n = c < 0 ? 0 : max(1, n);
+        // ceil(c / size), at least 1 (an empty sequence's workgroup writes its zero rows).
+        n = c < 0 ? 0 : max(1, split_count(c, size, __builtin_amdgcn_rcpf((float)size)));
         incl = wave_scan(n);
         const int count = __builtin_amdgcn_readlane(incl, 63);
         if (count <= workers) break;

@@ -12,4 +12,13 @@ namespace ak {
 // (one page per sequence), and 2^24 rows of 128 elements no longer fit an int.
 constexpr size_t page_row_offset(int t, int bs, int d) { return (size_t)(t & (bs - 1)) * d; }
 
+// ceil(c / size) for 0 <= c < 2^24 and size >= 32, from the hardware's
+// reciprocal of size.  With that and the product each off by a unit in the last
+// place the quotient is off by less than 1, so its whole part is the true one
+// or a neighbour: the remainder tells which, and one past it either way.
+constexpr int split_count(int c, int size, float reciprocal) {
+    const int n = (int)((float)c * reciprocal), r = c - n * size;
+    return n + (r > 0) + (r > size) - (r <= -size);
+}
+
 }  // namespace ak

@@ -23,6 +23,12 @@ def rcp(x, ulp):
     return np.nextafter(r, F(np.inf if ulp > 0 else -np.inf)) if ulp else r
 
 
+def split_count(c, size, reciprocal):
+    n = (c.astype(F) * reciprocal).astype(np.int64)
+    r = c - n * size
+    return n + (r > 0) + (r > size) - (r <= -size)
+
+
 def cut(lens, workers, cap, gran, ulp=0):
     c = np.minimum(np.maximum(np.asarray(lens, np.int64), 0), cap)
 
@@ -31,10 +37,7 @@ def cut(lens, workers, cap, gran, ulp=0):
 
     size = max(MIN_SPLIT, up(1 + int(F(c.sum() - 1) * rcp(workers, ulp))))
     for it in range(9):
-        n = (c.astype(F) * rcp(size, ulp)).astype(np.int64)
-        n += n * size < c
-        n -= (n - 1) * size >= c
-        n = np.maximum(1, n)
+        n = np.maximum(1, split_count(c, size, rcp(size, ulp)))
         count = int(n.sum())
         if count <= workers:
             break
@@ -57,6 +60,7 @@ def batches():
     yield [32768] + [1] * 31
     yield [0] * 7 + [5000]
     yield [(1 << 24) - 257, 1]
+    yield [14697473] + [1] * 15
     for _ in range(400):
         batch, high = int(rng.integers(2, MAX_BATCH + 1)), int(2 ** rng.uniform(10, 17))
         yield rng.integers(0 if rng.random() < 0.3 else 1, high + 1, batch).tolist()
@@ -67,7 +71,7 @@ def batches():
 def test_every_token_is_in_one_split(gran, ulp):
     for lens in batches():
         cap = -(-max(lens) // 256) * 256
-        for workers in (len(lens), len(lens) + 1, 2 * len(lens), 300):
+        for workers in (len(lens), len(lens) + 1, 2 * len(lens), 300, 512):
             segs, count, size = cut(lens, workers, cap, gran, ulp)
             assert count <= workers and size % gran == 0, (lens, workers)
             at = {}

@@ -9,9 +9,26 @@ from conftest import PKG_DIR
 
 CSRC = PKG_DIR / "attnkernels" / "csrc"
 WRAPPERS = """
+#include <cmath>
+
 #include "index_math.hpp"
 extern "C" {
 size_t page_row_offset(int t, int bs, int d) { return ak::page_row_offset(t, bs, d); }
+
+int split_count(int c, int size, float reciprocal) { return ak::split_count(c, size, reciprocal); }
+
+// Contexts just below, at and just above every multiple of size, with the
+// reciprocal a unit low, right and a unit high: the first wrong one, or -1.
+int first_wrong(int size) {
+    for (int u = -1; u <= 1; ++u) {
+        float r = 1.f / (float)size;
+        if (u) r = std::nextafter(r, u > 0 ? 2.f : 0.f);
+        for (int m = 0; m < (1 << 24); m += size)
+            for (int c = m - 2; c <= m + 2; ++c)
+                if (c >= 0 && c < (1 << 24) && ak::split_count(c, size, r) != (c + size - 1) / size) return c;
+    }
+    return -1;
+}
 }
 """
 
@@ -24,6 +41,8 @@ def lib(tmp_path_factory):
                     str(d / "w.so")], check=True)
     L = ctypes.CDLL(str(d / "w.so"))
     L.page_row_offset.argtypes, L.page_row_offset.restype = [ctypes.c_int] * 3, ctypes.c_size_t
+    L.split_count.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_float]
+    L.first_wrong.argtypes = [ctypes.c_int]
     return L
 
 
@@ -43,3 +62,9 @@ def test_the_whole_chunk_loops_use_it():
     text = (CSRC / "decode.hip").read_text()
     assert text.count("page_stride + page_row_offset(t, bs, D)") == 2
     assert "page_stride + (t & (bs - 1))" not in text
+
+
+def test_split_counts_are_exact_up_to_2_24_tokens(lib):
+    """Every multiple of a split size, and its neighbours, with a reciprocal off by a unit either way."""
+    for size in [*range(32, 4097, 32), *range(4096 + 64, 1 << 17, 4096 + 64), 29216, 33152, 1 << 20, (1 << 24) - 64, 1 << 24]:
+        assert lib.first_wrong(size) == -1, size
