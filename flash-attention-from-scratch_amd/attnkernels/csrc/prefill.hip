@@ -334,7 +334,11 @@ __device__ __forceinline__ void mask_tile(STile<D, NW, M>& s, int k0, int n, int
 }
 
 // Softmax state of the rows a lane owns: the subtracted (scaled, base-2) row
-// maximum m, starting at -inf, and the lane's share of the row sum l.
+// maximum m, starting at kNoMax, and the lane's share of the row sum l.  The
+// start is finite, so that keys that score -inf weigh 2^(-inf + |kNoMax|) = 0
+// before any other key is seen (and in a team that sees no other), as they do
+// after; a key of any other score overflows the sum there and moves m.
+constexpr float kNoMax = -3.4028234663852886e38f;  // the lowest float
 template <int QB>
 struct RowState {
     float m[QB];
@@ -461,7 +465,7 @@ __device__ __forceinline__ float chain_sum(const float (&c)[NCH]) {
 // Exponents checked after the fact instead of taking the tile maximum first:
 // P = 2^(S sl2 - m) is computed against the current subtracted maximum m, and
 // only if a lane's sum over key steps [C0, C1) reaches 2^14 (some P near the
-// top of fp16) or is not finite (the first tile, against m = -inf) does the
+// top of fp16) or is not finite (the first tile, against m = kNoMax) does the
 // wave come here.  All lanes of each such row then move m to the maximum of
 // those key steps, rescale O and l, and recompute P for them; rows that do not
 // move recompute the same P.  D = 128 checks whole tiles; D = 64 checks each
@@ -576,7 +580,7 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
     RowState<T::QB> st;
 #pragma unroll
     for (int qb = 0; qb < T::QB; ++qb) {
-        st.m[qb] = -INFINITY;  // the scaled row maxima subtracted so far
+        st.m[qb] = kNoMax;     // the scaled row maxima subtracted so far
         st.l[qb] = 0.f;        // this lane's share of the row sums
     }
 
@@ -791,7 +795,7 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
 #pragma unroll
             for (int qb = 0; qb < T::QB; ++qb) {
                 const float mk = src[PIECES * 4 * kWave + (2 * qb) * kWave + lane];
-                // The first team holds key 0, so its m is finite; one without keys has m = -inf and weighs 0.
+                // A team without keys (or with none above -inf) has m = kNoMax and weighs 0: its l and O are 0.
                 const float mx = fmaxf(st.m[qb], mk);
                 if (mx > st.m[qb]) move_max<D, NW, M>(st, o, qb, mx);
                 wo[qb] = exp2_fast(mk - mx);
@@ -813,7 +817,7 @@ __device__ __forceinline__ void prefill_qtile(const f16* __restrict__ qsrc, cons
 #pragma unroll
     for (int qb = 0; qb < T::QB; ++qb) {
         const float l_tot = row_sum<M>(st.l[qb]);
-        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        const float inv = 1.f / l_tot;  // a row whose every key scores -inf: 0 / 0
         const int qrow = qw0 + score_query<M>(qb, lane);
         if (qrow < n) {
             if constexpr (M == 32) {

@@ -144,6 +144,28 @@ def test_teams_when_the_maximum_sits_in_one_teams_keys():
             assert max_err(out, ref) < 2 * TOL[d]
 
 
+@pytest.mark.parametrize("d,n,dead", [(64, 257, (64, 128)), (128, 257, (32, 64)), (64, 300, (128, 192)),
+                                      (64, 2100, (64, 128)), (128, 700, (0, 96)), (64, 257, (0, 192)),
+                                      (128, 1100, (64, 128)), (128, 3100, (0, 64)), (64, 300, (0, 300))])
+@pytest.mark.parametrize("causal", [False, True])
+def test_keys_that_score_minus_infinity_weigh_nothing(d, n, dead, causal):
+    """A channel of -inf in K (q is 1 there) masks keys: all those of one team, of
+    the first tiles, or every key; only rows that see no other key are NaN."""
+    q, k, v = rand_qkv(1, 2, n, d, seed=n)
+    q[..., 0], k[..., 0] = 1, 0
+    k[:, :, dead[0]:dead[1], 0] = float("-inf")
+    out = run("wmma64", q, k, v, causal).float().cpu().numpy()
+    seen = np.ones((n, n), bool) if not causal else np.tri(n, dtype=bool)
+    seen[:, dead[0]:dead[1]] = False
+    rows = seen.any(1)
+    assert np.isnan(out[:, :, ~rows]).all()
+    for h in range(2):
+        s = q[0, h, :, 1:].double().numpy() @ k[0, h, :, 1:].double().numpy().T * d ** -0.5
+        s = np.where(seen, s, -np.inf)[rows]
+        w = np.exp(s - s.max(1, initial=-1e30, keepdims=True))
+        assert max_err(out[0, h, rows], w / w.sum(1, keepdims=True) @ v[0, h].double().numpy()) < TOL[d]
+
+
 def test_causal_first_row_is_v0():
     q, k, v = rand_qkv(1, 1, 128, 64, seed=5)
     for name in VARIANTS:
