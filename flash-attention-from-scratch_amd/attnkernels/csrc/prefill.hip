@@ -1014,7 +1014,9 @@ static PrefillPlan prefill_plan(const PrefillArgs& a) {
     const int64_t wg128 = tiles(128);
     PrefillPlan p{prefill_full(n, a.d, a.causal, a.bh), (int)a.bh};
     if (prefill_teams(n, a.d, a.causal, tiles(32), tiles(64), wg128, cus, p.kind) || !a.causal) return p;
-    if ((n + 127) / 128 * a.bh > INT_MAX / 2) return p;  // twice the workgroups of the pairs
+    // A launch holds fewer than 2^32 threads, and single tiles (256 threads per
+    // 128 rows, or 512 per 256) take twice as many as pairs.
+    if ((n + 255) / 256 * 512 * a.bh > UINT_MAX) return p;
     if (!a.cu) {
         p.kind = prefill_causal(n, a.d, a.bh, wg128, cus);
         // Groups of slices once their K and V no longer fit the XCDs' L2 (8 * 4 MB;

@@ -146,3 +146,15 @@ def test_capi_prefill_varlen():
     assert rc == 0, lib.ak_last_error()
     torch.cuda.synchronize()
     assert max_err(o, oracle.attention_varlen(q.numpy(), k.numpy(), v.numpy(), cu.numpy(), False)) < TOL[128]
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_varlen_with_a_loose_bound_on_many_sequences(d):
+    """The grid is sized by max_seqlen: at 4096 sequences x 4 heads and 2^17 rows, one
+    query tile per workgroup would take 2^32 threads, more than a launch holds."""
+    total, batch, h = 1 << 17, 1 << 12, 4
+    q, k, v, cu = (t.cuda() for t in packed([total // batch] * batch, h, 1, d, seed=d))
+    loose = ak.flash_attention_varlen(q, k, v, cu, total, causal=True)
+    tight = ak.flash_attention_varlen(q, k, v, cu, total // batch, causal=True)
+    assert max_err(loose[:4096], tight[:4096].float().cpu().numpy()) < TOL[d]
+    assert max_err(loose[-4096:], tight[-4096:].float().cpu().numpy()) < TOL[d]
