@@ -72,6 +72,18 @@ def test_odd_token_counts_and_skipped_halves_of_a_pair(d, skip):
     _check(key, value, kc0, vc0, kc, vc, slots)
 
 
+@pytest.mark.parametrize("tokens,hkv,d", [(4095, 8, 128), (4096, 8, 128), (4097, 8, 128), (16385, 2, 128), (8193, 8, 64),
+                                          (8191, 5, 40), (8193, 5, 40), (8193, 8, 96)])
+def test_both_sides_of_the_two_token_rule(tokens, hkv, d):
+    """One token per workgroup with stores into the L2, or two (an odd last one) with stores through it."""
+    key, value, kc, vc, slots = _case(tokens, hkv, d, tokens // 16 + 3, 16, torch.float16, seed=d)
+    slots[[0, tokens // 2, tokens - 2]] = -1
+    kc0, vc0 = kc.clone(), vc.clone()
+    ak.reshape_and_cache(key, value, kc, vc, slots)
+    torch.cuda.synchronize()
+    _check(key, value, kc0, vc0, kc, vc, slots)
+
+
 def test_padding_and_out_of_pool_slots_are_skipped():
     key, value, kc, vc, _ = _case(6, 8, 64, 4, 16, torch.float16, seed=3)
     slots = torch.tensor([5, -1, 63, 64, 1 << 40, 0], device="cuda", dtype=torch.int64)
