@@ -42,9 +42,9 @@ struct DecodeArgs {
     float* m_part;         // [B, hq, S]
     float* l_part;         // [B, hq, S]
     // One int per (sequence, kv head), zero on entry and left zero: when set
-    // (and 1 < S <= kFusedMaxSplits), the last split of each (sequence, kv
-    // head) to finish merges the partials in the decode kernel, with no reduce
-    // launch.  Null: the reduce kernel merges them.
+    // (and 1 < S <= kFusedMaxSplits, or the splits are balanced), the last split
+    // of each (sequence, kv head) to finish merges the partials in the decode
+    // kernel, with no reduce launch.  Null: the reduce kernel merges them.
     int32_t* counters;
     int64_t batch, hq, hkv, d, num_blocks, bs, max_blocks;
     int64_t partition, num_splits;
@@ -93,7 +93,7 @@ BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_
 // ak_paged_decode_noalloc, and its device address on the current GPU
 // (looked up once per device).
 constexpr size_t kDecodeScratchBytes = size_t(32) << 20;
-// Most splits merged in the decode kernel itself; more go to the reduce
+// Most fixed splits merged in the decode kernel itself; more go to the reduce
 // kernel, whose workgroups per row read them in parallel (measured at B = 1-4,
 // Hq = 32, Hkv = 8: 8-16 splits merged in the kernel save 1.5 us a call, 32
 // break even, 64 lose 3 us).

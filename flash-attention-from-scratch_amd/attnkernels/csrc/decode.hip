@@ -64,8 +64,8 @@ __device__ __forceinline__ f32x4 coherent_load4(const float* p) {  // 16-byte al
 template <int D, int G, int THREADS>
 __device__ __forceinline__ void merge_splits(const float* o_part, const float* m_part, const float* l_part,
                                              f16* out, size_t row0, size_t slot0, size_t hstride, int ns, int tid) {
-    // NB: loads per batch, enough for the most splits merged here in one batch,
-    // but no more than the kernel's main loop has registers for (8, or 16 for
+    // NB: loads per batch, enough for the most fixed splits in one batch (a long
+    // sequence's balanced ones take several), but no more than the kernel's main loop has registers for (8, or 16 for
     // the four- and eight-head kernels)
     constexpr int UNITS = G * D / 4, SG = THREADS / UNITS;
     constexpr int NB_CAP = G >= 4 ? 16 : 8, NB_ALL = (int)((kFusedMaxSplits + SG - 1) / SG);
@@ -195,6 +195,18 @@ __device__ __forceinline__ float wave_max(float x) {
 // (16 of 2000-20000, G = 4: 71.7 -> 72.0).
 constexpr int kDotGran = 64;
 
+// The most balanced splits of a sequence: one workgroup merges them, and with
+// more the merge of a long sequence among short ones takes longer than its
+// splits save.  One long sequence of eight, Hkv = 1, us a call with no bound /
+// 96 / 64 / 32 splits / fixed ones and the reduce kernel: G = 8, D = 128, 100000
+// tokens 37.0 / 28.4 / 31.9 / 47.9 / 32.9, 32768 tokens 22.0 / 19.2 / 17.9 /
+// 20.1 / 21.1, D = 64 22.8 / 16.9 / 18.4 / 26.7 / 19.0, 15.2 / 12.9 / 12.1 / 13.0 /
+// 13.0; G = 4, D = 128, 100000 tokens 23.7 / 20.9 / 23.8 / 34.9 / 26.8.  One head's
+// partials are merged by more threads each (16 sequences, 100000 tokens: 22.0 /
+// 24.2 / 30.2 / 49.3 / 27.5).
+template <int G>
+constexpr int kBalancedMostSplits = G == 1 ? 256 : 96;
+
 // Splits of about equal size, cut from the context lengths the kernel finds:
 // grid (kv head, workgroup), `workers` workgroups per kv head, one split each.
 // A fixed partition gives a ragged batch workgroups of very different
@@ -202,7 +214,8 @@ constexpr int kDotGran = 64;
 // ones finish.  Here every wave reads all the lengths (one load, a lane per
 // sequence), looks for the smallest split size (at least min_split tokens, a
 // multiple of GRAN) for which the sequences have at most `workers` splits in
-// all, and cuts each sequence into that many even ones.  Every workgroup of
+// all and none more than kBalancedMostSplits, and cuts each sequence into that
+// many even ones.  Every workgroup of
 // every kv head finds the same cut.  `order` holds flags:
 //   kLongestFirst: the splits run in the order of their lengths, in four
 //     classes by the quarters of the longest, so that a launch of more
@@ -216,10 +229,10 @@ __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_
     auto round_up = [](int x) { return (x + GRAN - 1) / GRAN * GRAN; };
     // No smaller size can do; even batches take this one.
     int size = max(min_split, round_up(1 + (int)((float)(total - 1) * __builtin_amdgcn_rcpf((float)workers))));
-    if (order & kEqualUncut) {
-        const int longest = (int)wave_max((float)max(c, 0));
-        if (!__builtin_amdgcn_ballot_w64(c >= 0 && c * 8 < longest * 7)) size = max(size, round_up(longest));
-    }
+    const int longest = (int)wave_max((float)max(c, 0));
+    size = max(size, round_up((longest + kBalancedMostSplits<G> - 1) / kBalancedMostSplits<G>));
+    if ((order & kEqualUncut) && !__builtin_amdgcn_ballot_w64(c >= 0 && c * 8 < longest * 7))
+        size = max(size, round_up(longest));
     int n, incl;
     for (int it = 0;; ++it) {
         // ceil(c / size), at least 1 (an empty sequence's workgroup writes its zero rows).
@@ -1363,8 +1376,9 @@ static bool one_round(int threads, int64_t wgs) {
 //     waves are further apart than two workgroups of 4 (12 x 4096 41.4 in 256,
 //     37.8 in 512; 16 of 512-8192 63.3, 56.1), but not below 96 of sequences
 //     times kv heads, where the merges cost more (4 x 8192: 26.3, 28.7).
-//   * More than 32 workgroups per sequence are too many for the merge in the
-//     decode kernel: fixed splits (2 x 100000, Hkv=1, G = 8: 28.2 us, 60.7 cut).
+//   * More than 32 workgroups per sequence on average are too many for the merge
+//     in the decode kernel: fixed splits (2 x 100000, Hkv=1, G = 8: 28.2 us, 60.7
+//     cut).  A sequence longer than the others gets up to kBalancedMostSplits.
 //   * One head at D = 128 takes as many rounds of 512 as give every sequence a
 //     workgroup (1.5 past 8192 tokens): four waves of 16 loads gain less from a
 //     cut than a second round costs (16 x 100-1200 tokens, Hkv=32: 39.0 us in

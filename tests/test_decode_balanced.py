@@ -16,6 +16,7 @@ BATCHES = {
     "skewed": [20000] + [3] * 15,
     "full": [1100 + 7 * i for i in range(64)],       # the most sequences, a lane each
     "two": [1, 4099],
+    "one long": [40000] + [30] * 7,                  # as many splits as one workgroup merges
     "empty": [0, 1500, 0, 2049, 0],                  # outside the >= 1 contract: zero rows
 }
 LONGEST = 1 << 16  # max_context_len given, so that even the small batches are cut by the kernel

@@ -29,13 +29,13 @@ def split_count(c, size, reciprocal):
     return n + (r > 0) + (r > size) - (r <= -size)
 
 
-def cut(lens, workers, cap, gran, ulp=0):
+def cut(lens, workers, cap, gran, ulp=0, most=96):
     c = np.minimum(np.maximum(np.asarray(lens, np.int64), 0), cap)
 
     def up(x):
         return (int(x) + gran - 1) // gran * gran
 
-    size = max(MIN_SPLIT, up(1 + int(F(c.sum() - 1) * rcp(workers, ulp))))
+    size = max(MIN_SPLIT, up(1 + int(F(c.sum() - 1) * rcp(workers, ulp))), up(-(-int(c.max()) // most)))
     for it in range(9):
         n = np.maximum(1, split_count(c, size, rcp(size, ulp)))
         count = int(n.sum())
@@ -79,6 +79,18 @@ def test_every_token_is_in_one_split(gran, ulp):
                 assert start == at.get(b, 0) and (end > start or lens[b] == 0), (lens, workers, b, s)
                 at[b] = end
             assert [at[b] for b in range(len(lens))] == lens, (lens, workers)
+
+
+@pytest.mark.parametrize("most", [96, 256])  # grouped-query heads, one head
+@pytest.mark.parametrize("gran", [32, 64])
+def test_no_sequence_has_more_splits_than_one_workgroup_merges(gran, most):
+    """One long sequence among short ones may take nearly every workgroup of a kv head."""
+    skewed = [([100000] + [500] * 7, 256), ([32768] + [500] * 7, 256), ([100000] + [500] * 15, 128),
+              ([100000] + [500] * 63, 512), ([32768] + [500] * 63, 1024), ([100000, 90000] + [1] * 14, 512)]
+    for lens, workers in [*skewed, *((b, 32 * len(b)) for b in batches())]:
+        segs, count, _ = cut(lens, workers, -(-max(lens) // 256) * 256, gran, most=most)
+        assert count <= workers and max(ns for _, _, ns, _, _ in segs) <= most, (lens, workers)
+    assert max(ns for _, _, ns, _, _ in cut(skewed[0][0], 256, 100352, gran, most=1 << 24)[0]) > 200
 
 
 @pytest.mark.parametrize("ulp", [-1, 0, 1])
