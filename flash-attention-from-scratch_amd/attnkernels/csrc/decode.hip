@@ -225,14 +225,17 @@ template <int G, int GRAN>
 __device__ __forceinline__ Segment balanced_segment(const int* __restrict__ ctx_lens, int kvh, int min_split,
                                                     int workers, int batch, int cap, int order, int lane) {
     const int c = lane < batch ? min(max(ctx_lens[lane], 0), cap) : -1;
+    const int longest = (int)wave_max((float)max(c, 0));
+    // Sequences of about one length stay whole where `order` says so: workgroup j takes sequence j.
+    if ((order & kEqualUncut) && !__builtin_amdgcn_ballot_w64(c >= 0 && c * 8 < longest * 7)) {
+        const int j = blockIdx.y;
+        return {j < batch ? j : -1, 0, 1, 0, j < batch ? __builtin_amdgcn_readlane(c, j) : 0, 0, (size_t)workers};
+    }
     const int total = __builtin_amdgcn_readlane(wave_scan(max(c, 0)), 63);
     auto round_up = [](int x) { return (x + GRAN - 1) / GRAN * GRAN; };
     // No smaller size can do; even batches take this one.
     int size = max(min_split, round_up(1 + (int)((float)(total - 1) * __builtin_amdgcn_rcpf((float)workers))));
-    const int longest = (int)wave_max((float)max(c, 0));
     size = max(size, round_up((longest + kBalancedMostSplits<G> - 1) / kBalancedMostSplits<G>));
-    if ((order & kEqualUncut) && !__builtin_amdgcn_ballot_w64(c >= 0 && c * 8 < longest * 7))
-        size = max(size, round_up(longest));
     int n, incl;
     for (int it = 0;; ++it) {
         // ceil(c / size), at least 1 (an empty sequence's workgroup writes its zero rows).
