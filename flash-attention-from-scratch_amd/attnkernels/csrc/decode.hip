@@ -1362,8 +1362,8 @@ static bool one_round(int threads, int64_t wgs) {
 //     31.1 fixed, 23.3 balanced).
 //   * More than 64 sequences do not fit one load of lengths by a wave; a batch
 //     that large fills the GPU by itself.
-//   * Workgroups in whole rounds of the GPU (one 8-wave workgroup per CU, two
-//     or more of 4 waves), because HBM idles in a partial one: 384 workgroups
+//   * Workgroups in whole rounds of one per CU (an 8-wave workgroup, or two or
+//     more of 4 waves), because HBM idles in a partial one: 384 workgroups
 //     measure 10-25% behind 256 and 512.
 //   * 1.7 of them per sequence where the batch itself is up to 512: with fewer
 //     the longest sequences cannot be cut (24 of 512-8192 tokens, Hkv=8, in 256
@@ -1373,35 +1373,51 @@ static bool one_round(int threads, int64_t wgs) {
 //     512, 57.5 in 1024).
 //     Past 512, 1.1 of them (1.5 for contexts past 8192: one long sequence
 //     among short ones): the order below does the balancing.
+//   * 3.2 where the longest context is 2048 times the batch or more (from 8
+//     sequences): a long one among short ones, which take a workgroup each and
+//     leave it the rest (16, one of 100000, Hkv=8, in 256 and 512, fixed: Hq=64,
+//     D=64 55.6, 46.8, 49.0; Hq=8, D=64 49.2, 39.7, 41.6; 8, Hkv=32, Hq=128, in
+//     512 and 1024, fixed: 306, 281, 286).
 //   * Up to 1024 workgroups, the first size of which equal sequences, each cut
-//     alike, fill more than three quarters (24 x 4096, Hq=32: 68.2 in 512, 67.0
-//     in 768).  Eight heads at D = 128 start at 512: the matrix-core kernel's 8
-//     waves are further apart than two workgroups of 4 (12 x 4096 41.4 in 256,
-//     37.8 in 512; 16 of 512-8192 63.3, 56.1), but not below 96 of sequences
-//     times kv heads, where the merges cost more (4 x 8192: 26.3, 28.7).
+//     alike, keep more than three quarters of the rounds they make busy (24 x
+//     4096, Hq=32: 68.2 in 512, 67.0 in 768; 56 x 2048, Hq=64, in 768, where they
+//     stay whole and fill 448 of 512, 76.8, in 1024 87.4, fixed 85.8).  Eight
+//     heads at D = 128 start at 512: the matrix-core kernel's 8 waves are further
+//     apart than two workgroups of 4 (12 x 4096 41.4 in 256, 37.8 in 512; 16 of
+//     512-8192 63.3, 56.1), but not below 96 of sequences times kv heads, where
+//     the merges cost more (4 x 8192: 26.3, 28.7).
 //   * More than 32 workgroups per sequence on average are too many for the merge
 //     in the decode kernel: fixed splits (2 x 100000, Hkv=1, G = 8: 28.2 us, 60.7
 //     cut).  A sequence longer than the others gets up to kBalancedMostSplits.
-//   * One head at D = 128 takes as many rounds of 512 as give every sequence a
-//     workgroup (1.5 past 8192 tokens): four waves of 16 loads gain less from a
-//     cut than a second round costs (16 x 100-1200 tokens, Hkv=32: 39.0 us in
-//     512 workgroups, 43.8 in up to 1024).  Where that leaves less than an
-//     eighth in a single round, there is nothing to balance and the fixed
-//     splits start sooner.
+//   * One head at D = 128 runs two workgroups of 4 waves per CU and starts at 512;
+//     from there it takes the size that equal sequences fill best (Hkv=8, in
+//     512, 768 and 1024, fixed: 22 x 4096 68.1, 60.8, 66.7, 60.6; 40 x 4096 122.6,
+//     114.1, 108.7, 105.5; 33 x 4096 117.4, 108.1, 97.5, 95.6; 40 of 512-8192 130,
+//     123, 119, 123), but stays in 512 where three quarters of them are busy (24
+//     of 512-8192: 61.0, 63.3, 60.9, 73.2).  Shorter contexts pay more for a
+//     second round (up to 2048 tokens 1.3 workgroups per sequence: 24 x 1500,
+//     Hkv=16 49.6 in 512, 54.3 in 768), longer ones gain more (56 of 512-8192 in
+//     768 and 1024: 178, 164), a lone long one most, from 4096 times the batch on
+//     (16, one of 100000, Hkv=16, in 512 and 1536, fixed: 173, 141, 155).  Within
+//     an eighth of 512 and up to 8192 tokens the fixed splits serve: they start
+//     sooner (16 x 100-1200 tokens, Hkv=32: 35.1, in 1024 36.3).  Past 512, whole
+//     rounds of 512 with a workgroup per sequence (1.5 past 8192 tokens).
 //   * Past 512 workgroups the longest splits run first, in four classes (a rank
 //     of each by comparisons with all others costs 2-5 us at 64 sequences, the
 //     classes 0.3): 64 of 1-4096 tokens, Hkv=32 368.9 -> 346.2, 32 of 100-8192
 //     429.8 -> 379.0; 56 of 512-8192, Hq=64, Hkv=8 193.3 -> 169.9.
 //   * Sequences of about one length stay whole where the batch fills two rounds
-//     or more: 64 x 4096, Hkv=8: Hq=32 169.9 -> 164.0, Hq=64 176.0 -> 163.7
-//     (fixed splits 163.6 and 161.6).
+//     or more, found before any cut: 64 x 4096, Hkv=8: Hq=32 169.9 -> 164.0, Hq=64
+//     176.0 -> 161.2 (fixed splits 163.6 and 160.0).
 // Measured against fixed splits of decode_partition (us a call, back to back;
 // Hq=32, Hkv=8, D=128 unless noted): 16 x 8192 89.3 -> 84.4; 16 ragged 512-8192
 // 63.4 -> 52.9, with Hq=64 76.8 -> 57.3; 24 of them 103.4 -> 92.8, 40 127.7 ->
 // 118.7; 64 of 1-8192 197.8 -> 182.0, with Hq=64 235.7 -> 193.7; 8 of 500-32000,
 // Hq=16 114.1 -> 98.0; 8 x 32768, Hkv=32 678 -> 652 (D=64: 366 -> 331).
-// Behind them: 22 x 4096 62.3 -> 63.0, 33 x 4096 98.2 -> 100.9, 24 x 4096, Hq=64
-// 70.6 -> 72.0, 64 x 2048, Hq=64 82.0 -> 84.5.
+// Behind them by what the cut costs (0.3-1 us) or where equal sequences fill no
+// size well: 22 x 4096 60.8 -> 61.9, with Hq=64 66.3 -> 67.9; 24 x 4096, Hq=64
+// 69.4 -> 70.9; 33 x 4096 96.9 -> 99.5, with Hq=64 104.6 -> 108.4, Hq=8 95.6 ->
+// 98.0; 40 x 4096, Hq=64 114.8 -> 119.0; 64 x 2048, Hq=64 80.9 -> 82.3.
 BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_t d, int64_t max_ctx, int64_t cap) {
     if (batch < 2 || batch > kBalancedMaxBatch || max_ctx <= 1024 || cap >= (int64_t(1) << 24) ||
         batch * hkv * max_ctx * d * 4 < (int64_t(64) << 20))
@@ -1411,28 +1427,29 @@ BalancedPlan decode_balanced_plan(int64_t batch, int64_t hq, int64_t hkv, int64_
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
     const bool one_head = hq == hkv && d == 128;
-    const int64_t round = one_head ? 2 * cus : cus;
-    int64_t k, workers;
-    if (one_head) {
-        const int64_t need = batch + (max_ctx > 8192 ? batch / 2 : 0);
-        k = (need * hkv + round - 1) / round;
-        workers = k * round / hkv;
+    const int64_t wgs = batch * hkv;
+    int64_t k;  // rounds of one workgroup per CU
+    if (wgs > 2 * cus) {
+        if (one_head) k = (wgs + (max_ctx > 8192 ? batch / 2 * hkv : 0) + 2 * cus - 1) / (2 * cus) * 2;
+        else k = (wgs * (max_ctx > 8192 ? 15 : 11) + 10 * cus - 1) / (10 * cus);
     } else {
-        const bool cut = batch * hkv <= 2 * cus;
-        k = (batch * hkv * (cut ? 17 : max_ctx > 8192 ? 15 : 11) + 10 * cus - 1) / (10 * cus);
-        if (cut && hq == 8 * hkv && d == 128 && batch * hkv * 8 >= 3 * cus) k = std::max<int64_t>(k, 2);
-        for (int64_t i = k; cut && i <= std::max<int64_t>(k, 4); ++i) {
-            const int64_t w = i * round / hkv;
-            if (w / batch * batch * 4 > w * 3) {
-                k = i;
-                break;
-            }
+        if (one_head && max_ctx <= 8192 && wgs * 9 > 16 * cus) return {0, 0};
+        const bool lone = batch >= 8 && max_ctx >= (one_head ? 4096 : 2048) * batch;
+        const int64_t tenths = lone ? (one_head ? 50 : 32) : !one_head ? 17 : max_ctx <= 2048 ? 13 : max_ctx <= 4096 ? 17 : 18;
+        k = (wgs * tenths + 10 * cus - 1) / (10 * cus);
+        if (one_head || (hq == 8 * hkv && d == 128 && wgs * 8 >= 3 * cus)) k = std::max<int64_t>(k, 2);
+        if (one_head && lone) k = (k + 1) / 2 * 2;
+        int64_t best = 0;
+        for (int64_t i = k, last = std::max<int64_t>(k, 4); i <= last; ++i) {
+            const int64_t used = i * cus / hkv / batch * wgs, rounds = (used + cus - 1) / cus;
+            const int64_t fill = rounds ? used * 1000 / (rounds * cus) : 0;  // by equal sequences, each cut alike
+            if (fill > best) best = fill, k = i;
+            if (one_head ? fill >= (i == 2 ? 750 : 1000) : fill > 750) break;
         }
-        workers = k * round / hkv;
     }
-    if (batch * hkv <= round && workers * 8 < batch * 9) return {0, 0};
+    const int64_t workers = k * cus / hkv;
     if (workers > kFusedMaxSplits * batch) return {0, 0};
-    const bool rounds = !one_head && batch * hkv >= 2 * cus && batch * hkv % cus == 0;
+    const bool rounds = !one_head && wgs >= 2 * cus && wgs % cus == 0;
     return {workers, (workers * hkv > 2 * cus ? kLongestFirst : 0) | (rounds ? kEqualUncut : 0)};
 }
 

@@ -173,6 +173,40 @@ def test_rule(lib):
     assert workers(lib, 16, 32, 8, 128, 8192) == 32 and workers(lib, 16, 32, 32, 128, 8192) == 0 and workers(lib, 8, 32, 32, 128, 8192) == 16
 
 
+@pytest.mark.parametrize("batch,hq,hkv,d,max_ctx,per_cu", [
+    # the first size that equal sequences keep three quarters busy, cut or whole
+    (16, 32, 8, 128, 8192, 1), (22, 32, 8, 128, 4096, 3), (33, 64, 8, 128, 4096, 4), (40, 32, 8, 128, 4096, 3),
+    (52, 64, 8, 128, 3000, 3), (56, 64, 8, 128, 2048, 3), (57, 64, 8, 128, 2048, 4), (64, 32, 8, 128, 4096, 4),
+    # a lone long sequence, and just not
+    (16, 8, 8, 64, 32768, 2), (16, 8, 8, 64, 32767, 1), (8, 128, 32, 128, 16384, 4), (8, 128, 32, 128, 16383, 2),
+    (7, 128, 32, 128, 100000, 2),
+    # one head at D = 128: from two, the best filled size, fewer for short contexts, fixed when nearly full
+    (12, 8, 8, 128, 4096, 2), (22, 8, 8, 128, 4096, 3), (24, 8, 8, 128, 8192, 2), (33, 8, 8, 128, 4096, 4), (40, 8, 8, 128, 4096, 4),
+    (24, 16, 16, 128, 2048, 2), (24, 16, 16, 128, 2049, 3), (56, 8, 8, 128, 4096, 3), (56, 8, 8, 128, 4097, 4),
+    (56, 8, 8, 128, 8192, 4), (57, 8, 8, 128, 8192, 0), (57, 8, 8, 128, 8193, 4), (16, 16, 16, 128, 65536, 6), (16, 16, 16, 128, 65535, 2),
+    # past 512 sequences times kv heads
+    (64, 64, 16, 128, 4096, 5), (64, 64, 16, 128, 8193, 6), (33, 16, 16, 128, 4096, 4), (64, 32, 32, 128, 8193, 12)])
+def test_sizes_of_the_rule(lib, batch, hq, hkv, d, max_ctx, per_cu):
+    """Workgroups per CU (256 of them) that the rule launches for sizes on both sides of its lines."""
+    assert workers(lib, batch, hq, hkv, d, max_ctx) == per_cu * 256 // hkv
+
+
+def test_every_sequence_has_a_workgroup_and_a_long_one_is_cut(lib):
+    for batch in range(2, MAX_BATCH + 1):
+        for hkv in (1, 2, 3, 4, 5, 7, 8, 12, 16, 32, 40, 100, 256, 300, 513):
+            for g in (1, 4, 8):
+                for d in (64, 128):
+                    for ctx in (1025, 4096, 8193, 200000):
+                        w = workers(lib, batch, g * hkv, hkv, d, ctx)
+                        if w and batch * hkv <= 512:
+                            lens = [ctx] + [500] * (batch - 1)
+                            segs, count, _ = cut(lens, w, ctx + 255, 64)
+                            assert count <= w
+                            if ctx > 4096:
+                                assert segs[0][2] >= 2, (batch, hkv, g, d, ctx, w)
+                        assert w == 0 or w >= batch
+
+
 def test_refused_calls(lib):
     fake = ctypes.c_void_p(4096)
 
