@@ -10,6 +10,7 @@
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -36,23 +37,50 @@ void* stream_of(const torch::Tensor& t) {
     return at::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
+// The stream capture that calls on `stream` are recorded into, 0: none.
+unsigned long long capture_id(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) return 0;
+    return status == hipStreamCaptureStatusNone ? 0 : id;
+}
+
 // Split counters of the decode kernels' in-kernel merge, one array per
 // (device, stream): zeroed when allocated, and every decode call leaves its
 // counters at zero, so the calls on a stream (which run in order) share it.
-// A stream that needs more counters gets a new, larger array; the smaller one
-// is kept, because a captured graph may still use it.
+// The calls recorded into a graph share another one, per stream and capture:
+// what zeroes it is recorded before them, so each replay starts from zeros
+// whatever has used that memory since (graphs that share a memory pool reuse
+// each other's), and two graphs never share counters.  It is let go when the
+// stream records the next graph; an array grown during a capture is kept that long too.
 // The cache is never destroyed: its tensors would otherwise be freed during
 // static destruction, after torch's allocator or the HIP runtime may be gone.
 torch::Tensor split_counters(const torch::Tensor& q, int64_t n) {
+    struct Arrays {
+        torch::Tensor eager;
+        unsigned long long capture = 0;
+        std::vector<torch::Tensor> captured;
+    };
     static std::mutex mu;
-    static auto* cache = new std::map<std::pair<int, void*>, std::vector<torch::Tensor>>();
+    static auto* cache = new std::map<std::pair<int, void*>, Arrays>();
+    void* const stream = stream_of(q);
+    const unsigned long long capture = capture_id(stream);
     std::lock_guard<std::mutex> lock(mu);
-    auto& arrays = (*cache)[{(int)q.device().index(), stream_of(q)}];
-    if (arrays.empty() || arrays.back().numel() < n) {
-        const int64_t grow = arrays.empty() ? 0 : 2 * arrays.back().numel();
-        arrays.push_back(torch::zeros({std::max(n, std::max<int64_t>(grow, 4096))}, q.options().dtype(torch::kInt)));
+    auto& arrays = (*cache)[{(int)q.device().index(), stream}];
+    if (capture != 0 && arrays.capture != capture) {
+        arrays.captured.clear();
+        arrays.capture = capture;
     }
-    return arrays.back();
+    torch::Tensor last = capture == 0                ? arrays.eager
+                         : arrays.captured.empty() ? torch::Tensor()
+                                                     : arrays.captured.back();
+    if (!last.defined() || last.numel() < n) {
+        const int64_t grow = last.defined() ? 2 * last.numel() : 0;
+        last = torch::zeros({std::max(n, std::max<int64_t>(grow, 4096))}, q.options().dtype(torch::kInt));
+        if (capture == 0) arrays.eager = last;
+        else arrays.captured.push_back(last);
+    }
+    return last;
 }
 
 }  // namespace
