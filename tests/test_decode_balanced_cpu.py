@@ -29,15 +29,22 @@ def split_count(c, size, reciprocal):
     return n + (r > 0) + (r > size) - (r <= -size)
 
 
-def cut(lens, workers, cap, gran, ulp=0, most=96):
+def rounded_up_count(c, size, reciprocal):
+    """The planted mistake: a float ceiling with no correction."""
+    return np.ceil(c.astype(F) * reciprocal).astype(np.int64)
+
+
+def cut(lens, workers, cap, gran, ulp=0, most=96, equal_uncut=False, count_splits=split_count):
     c = np.minimum(np.maximum(np.asarray(lens, np.int64), 0), cap)
+    if equal_uncut and (c * 8 >= c.max() * 7).all():
+        return [(b, 0, 1, 0, int(n)) for b, n in enumerate(c)], len(lens), max(MIN_SPLIT, int(c.max()))
 
     def up(x):
         return (int(x) + gran - 1) // gran * gran
 
     size = max(MIN_SPLIT, up(1 + int(F(c.sum() - 1) * rcp(workers, ulp))), up(-(-int(c.max()) // most)))
     for it in range(9):
-        n = np.maximum(1, split_count(c, size, rcp(size, ulp)))
+        n = np.maximum(1, count_splits(c, size, rcp(size, ulp)))
         count = int(n.sum())
         if count <= workers:
             break
@@ -74,11 +81,25 @@ def test_every_token_is_in_one_split(gran, ulp):
         for workers in (len(lens), len(lens) + 1, 2 * len(lens), 300, 512):
             segs, count, size = cut(lens, workers, cap, gran, ulp)
             assert count <= workers and size % gran == 0, (lens, workers)
-            at = {}
-            for b, s, ns, start, end in segs:
-                assert start == at.get(b, 0) and (end > start or lens[b] == 0), (lens, workers, b, s)
-                at[b] = end
-            assert [at[b] for b in range(len(lens))] == lens, (lens, workers)
+            assert tiles(lens, segs), (lens, workers)
+
+
+def tiles(lens, segs):
+    """Whether the splits tile every context, and each holds a token (or its sequence none)."""
+    at = {}
+    for b, s, ns, start, end in segs:
+        if start != at.get(b, 0) or (end <= start and lens[b] > 0):
+            return False
+        at[b] = end
+    return [at[b] for b in range(len(lens))] == list(lens)
+
+
+def test_about_equal_sequences_stay_whole_where_the_launch_says_so():
+    for lens, whole in (([2048, 1792] + [1900] * 62, True), ([2048, 1791] + [1900] * 62, False), ([0] * 64, True),
+                        ([0] + [5] * 63, False), ([4096] * 32, True)):
+        segs, count, _ = cut(lens, 2 * len(lens), 4096, 32, equal_uncut=True)
+        assert tiles(lens, segs) and count <= 2 * len(lens)
+        assert (all(ns == 1 for _, _, ns, _, _ in segs) and count == len(lens)) == (whole or max(lens) <= MIN_SPLIT)
 
 
 @pytest.mark.parametrize("most", [96, 256])  # grouped-query heads, one head
@@ -120,11 +141,10 @@ def test_even_batches_are_cut_evenly():
 
 
 def test_a_cut_that_rounds_up_its_count_is_caught():
-    """With a float ceiling alone (no step of correction) 2 * size tokens can count as 3 splits, one of them empty."""
-    size, ctx = 128, 256
-    n = int(np.ceil(F(ctx) * rcp(size, 1)))
-    length = -(-(-(-ctx // n)) // 128) * 128
-    assert n == 3 and (n - 1) * length >= ctx
+    """With a float ceiling alone 2 * size tokens can count as 3 splits, one of them empty."""
+    lens = [2 * MIN_SPLIT] * 2
+    assert tiles(lens, cut(lens, 8, 512, 128, ulp=1)[0])
+    assert not tiles(lens, cut(lens, 8, 512, 128, ulp=1, count_splits=rounded_up_count)[0])
 
 
 @pytest.fixture(scope="module")

@@ -72,6 +72,27 @@ def decode_calls():
         yield lambda b=bad: ak.paged_decode(*b, 300)
 
 
+def balanced_calls():
+    """Large enough at the longest context given that the splits are balanced, as each route reaches them."""
+    kc, vc, bt, cl = oracle.make_paged_cache([3000, 40, 1700, 1], 8, 128, block_size=16, extra_blocks=1, seed=0)
+    kc, vc, bt, cl = (torch.from_numpy(a).cuda() for a in (kc, vc, bt, cl))
+    q = rand(4, 16, 128)
+    for args in ((bt, cl), (bt.long(), cl), (bt, cl.long())):
+        yield lambda a=args: ak.paged_decode(q, kc, vc, *a, 16000)
+
+
+def test_balanced_routes_agree(monkeypatch):
+    """One answer for tables and lengths of either integer type, by either route."""
+    answers = [f() for f in balanced_calls()] + [checked(monkeypatch, f) for f in balanced_calls()]
+    assert all(same(a, answers[0]) for a in answers)
+    fixed = ak.load_extension().paged_decode  # other sums: the default did take balanced splits
+    kc, vc, bt, cl = (torch.from_numpy(a).cuda() for a in oracle.make_paged_cache([3000, 40, 1700, 1], 8, 128, block_size=16,
+                                                                                 extra_blocks=1, seed=0))
+    part = ak.decode_partition(4, 8, 16000)
+    other = fixed(rand(4, 16, 128), kc, vc, bt, cl, 16000, 128 ** -0.5, part)
+    assert not torch.equal(other, answers[0]) and (other - answers[0]).abs().max() < 1e-3
+
+
 @pytest.mark.parametrize("calls", [prefill_calls, decode_calls])
 def test_answers_and_errors_are_those_of_the_checked_route(calls, monkeypatch):
     for i, fn in enumerate(calls()):
@@ -103,6 +124,18 @@ def test_only_plain_tensors_take_it():
     ext = ak.load_extension()
     q = rand(1, 2, 16, 64)
     assert isinstance(ext.plain_prefill(q, q, q, False, None, False), torch.Tensor)
+    assert isinstance(ext.plain_prefill(q, q[:, :1], q[:, :1], True, 0.5, True), torch.Tensor)
+    x, cu = rand(20, 4, 64), torch.tensor([0, 7, 20], dtype=torch.int32, device="cuda")
+    assert isinstance(ext.plain_varlen(x, x, x, cu, 13, True, None), torch.Tensor)
+    assert ext.plain_varlen(x, x, x, cu.long(), 13, True, None) is None
+    kc, vc, bt, cl = (torch.from_numpy(a).cuda() for a in oracle.make_paged_cache([40, 300], 2, 64, block_size=16, seed=0))
+    qd = rand(2, 4, 64)
+    for part in (None, 256):
+        assert isinstance(ext.plain_decode(qd, kc, vc, bt, cl, 300, None, part, ak.decode_partition), torch.Tensor)
+        assert ext.plain_decode(qd, kc, vc, bt.long(), cl, 300, None, part, ak.decode_partition) is None
+    key, slots = rand(5, 2, 64), torch.arange(5, device="cuda")
+    assert ext.plain_write(key, key, kc, vc, slots) is True
+    assert ext.plain_write(key, key, kc, vc, slots.int()) is False
     assert ext.plain_prefill(q.cpu(), q, q, False, None, False) is None
     assert ext.plain_prefill(q, q, q, 1, None, False) is None
 

@@ -113,9 +113,11 @@ def test_mfma_shape_boundaries(causal, h, n):
 
 @pytest.mark.parametrize("d,causal,h,n", [
     # teams of one wave x 4, two x 4 and four x 2: tiles without keys for a team, ragged row and key tiles
-    (64, False, 8, 257), (128, True, 4, 97), (64, True, 3, 65), (64, False, 5, 1537), (128, False, 10, 801),
+    (64, False, 8, 257), (128, True, 4, 225), (64, True, 3, 193), (64, False, 5, 1537), (128, False, 10, 801),
     (64, True, 6, 2049), (128, True, 6, 3073), (64, False, 14, 2047), (64, True, 30, 1023), (128, False, 8, 3073),
-    (128, True, 12, 3100), (64, True, 300, 1),
+    (128, True, 12, 3100),
+    # below them: up to 192 rows one tile per workgroup, up to 128 no order among them
+    (128, True, 4, 97), (64, True, 3, 65), (64, True, 300, 1), (128, True, 4, 192),
     # single tiles: one group of slices, several with a smaller last one, 8 waves, 16x16 MFMAs
     (128, True, 64, 700), (64, True, 70, 385), (128, True, 520, 257), (64, True, 24, 4097), (128, True, 26, 3585),
     # pairs between three and four workgroups' worth of tiles per CU
@@ -235,6 +237,18 @@ def test_workgroup_sizes_agree(causal, n, d):
     ref = oracle.attention_fp32(q[:, :2].numpy(), k[:, :2].numpy(), v[:, :2].numpy(), causal)
     assert max_err(small, ref) < TOL[d]
     assert max_err(big[:, :2], ref) < TOL[d]
+
+
+@pytest.mark.parametrize("causal,n,d", [(True, 300, 128), (False, 800, 128), (True, 4000, 128), (True, 300, 64),
+                                        (False, 800, 64)])
+def test_heads_alone_and_among_others_agree_to_rounding(causal, n, d):
+    """Outside the lengths of the test above, small grids deal a row's key tiles to teams
+    of waves, or take another MFMA shape: other orders of the same sums."""
+    q, k, v = rand_qkv(1, 64, n, d, seed=n + d)
+    big = run("wmma64", q, k, v, causal)
+    small = run("wmma64", q[:, :2], k[:, :2], v[:, :2], causal)
+    ref = oracle.attention_fp32(q[:, :2].numpy(), k[:, :2].numpy(), v[:, :2].numpy(), causal)
+    assert max_err(small, ref) < TOL[d] and max_err(big[:, :2], ref) < TOL[d]
 
 
 # ---------------------------------------------------- BASELINE full sizes --
