@@ -13,7 +13,8 @@ The same line carries, under ``workloads``, the other BASELINE configs measured
 the same way: non-causal prefill, the N=8191 variant, the two
 paged split-K decode configs in KV GB/s with the reference's byte convention
 sum(ctx)*Hkv*D*2*2 (bench/bench.py:199-200), two grouped-query decode layers (4
-and 8 query heads per kv head) at the library's default partition, the paged
+and 8 query heads per kv head) with no partition given (the library's own
+splits: balanced, or of decode_partition's tokens), the paged
 cache writer (K/V rows read + written, GB/s), and a packed variable-length GQA
 prefill.
 
@@ -200,15 +201,28 @@ def prefill_case(b, h, n, d, causal, steps, warmup, seed=0):
     return res
 
 
+def balanced_workgroups(batch, hq, hkv, d, max_ctx, partition):
+    """Workgroups per kv head of the balanced splits that paged_decode takes when no
+    partition is given, 0 where splits of `partition` tokens serve these sizes."""
+    import ctypes
+
+    from attnkernels import build as akbuild
+
+    size = ctypes.CDLL(str(akbuild.LIB)).ak_paged_decode_balanced_workspace_size
+    size.argtypes, size.restype = [ctypes.c_int64] * 6, ctypes.c_size_t
+    return size(batch, hq, hkv, d, max_ctx, partition) // (hq * (d + 2) * 4)
+
+
 def decode_case(lens, hkv, d, bs, partition, steps, warmup, seed=0, hq=None):
+    """partition: tokens per split, or None for the call as the library splits it by itself."""
     import numpy as np
     import torch
 
     import attnkernels as ak
 
     hq = hkv if hq is None else hq
-    if partition is None:  # the library's default split rule
-        partition = ak.decode_partition(len(lens), hkv, max(lens))
+    fixed = ak.decode_partition(len(lens), hkv, max(lens)) if partition is None else partition
+    balanced = balanced_workgroups(len(lens), hq, hkv, d, max(lens), fixed) if partition is None else 0
     nblk = [-(-c // bs) for c in lens]
     pool = -(-sum(nblk) * 11 // 10)
     rng = np.random.default_rng(seed)
@@ -241,9 +255,12 @@ def decode_case(lens, hkv, d, bs, partition, steps, warmup, seed=0, hq=None):
     del out, kseq, vseq
     t = timed_steps(fn, steps, warmup)
     nbytes = decode_kv_bytes(lens, hkv, d)
-    res = dict(workload=f"paged decode B={len(lens)} Hq={hq} Hkv={hkv} D={d} bs={bs} P={partition} "
+    splits = (f"balanced splits, {balanced} workgroups per kv head" if balanced
+              else f"P={fixed}" + (" (default)" if partition is None else ""))
+    res = dict(workload=f"paged decode B={len(lens)} Hq={hq} Hkv={hkv} D={d} bs={bs} {splits} "
                         f"sum_ctx={sum(lens)} max_ctx={max_ctx}",
-               **timing_fields(t, steps, nbytes, "GB/s"), bytes_per_step=nbytes, splits=-(-max_ctx // partition),
+               **timing_fields(t, steps, nbytes, "GB/s"), bytes_per_step=nbytes,
+               splits=balanced // len(lens) if balanced else -(-max_ctx // fixed),
                max_abs_err=float(f"{err:.3g}"))
     del kc, vc, q
     torch.cuda.empty_cache()
@@ -465,9 +482,9 @@ def main():
         "decode_ragged64_d128": lambda: decode_case(lens4, 32, 128, 16, 512, K, W),
         "decode_long8_d128": lambda: decode_case([32768] * 8, 32, 128, 16, 256, K, W),
         "decode_long8_d64": lambda: decode_case([32768] * 8, 32, 64, 16, 256, K, W),
-        # a Llama-3-8B-like decode layer: 4 query heads per kv head, the default partition
+        # a Llama-3-8B-like decode layer: 4 query heads per kv head, no partition given
         "decode_gqa16_d128": lambda: decode_case([8192] * 16, 8, 128, 16, None, K, W, hq=32),
-        # 8 query heads per kv head (the heaviest head group the kernels take), default partition
+        # 8 query heads per kv head (the heaviest head group the kernels take), no partition given
         "decode_g8_d128": lambda: decode_case([8192] * 8, 8, 128, 16, None, K, W, hq=64),
         # packed prompts of mixed lengths, 4 query heads per kv head, no padding
         "prefill_varlen_gqa": lambda: varlen_case(lensv, 32, 8, 128, True, K, W),

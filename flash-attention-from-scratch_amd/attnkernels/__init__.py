@@ -88,6 +88,10 @@ def naive_attention(q, k, v, causal=False, scale=None):
 def flash_attention(q, k, v, causal=False, scale=None, variant="wmma", block_n=None):
     """Tiled attention with online softmax. q, k, v: fp16 [B, H, N, D], D in {64, 128}.
 
+    The order in which a row's keys are summed, and with it the last bit of a
+    result, depends on B * H where small grids split the work otherwise than large
+    ones do: at D = 64 for all N, at D = 128 for N up to 1024 and from 3072 on.
+
     variant: "simt" or "wmma" (both run the gfx950 MFMA kernel).
     block_n: key-tile width accepted by "wmma" (32 or 64), as in the reference.
     Reference: attnkernels/__init__.py:71-85.
@@ -113,7 +117,8 @@ def _sm_count(device_index):
     return torch.cuda.get_device_properties(device_index).multi_processor_count
 
 
-# Split-count target of decode_partition.  The reference's rule aims at 4
+# Split-count target of decode_partition, which paged_decode falls back on where
+# it does not balance the splits itself.  The reference's rule aims at 4
 # blocks per SM (attnkernels/__init__.py:94-98, tuned on a T4).  The partition
 # is chosen from max_context_len alone (reading the lengths would cost a host
 # sync), so the rule must hold for uniform, mixed-length and skewed batches.
@@ -145,10 +150,12 @@ def _sm_count(device_index):
 #     the best), uniform and mixed ones at 1024-16384 (512 reads 79-94% over
 #     three runs); a floor of 1 chunk would cost the uniform ones 14-26%;
 #   * tokens per split a power-of-two number of chunks.
-# Together they reach 97% of the best partition on average and 88% in the
-# worst case in the committed ablation (without the long-context clause 95%
+# Together they reach 97% of the best partition on average and 87% in the
+# worst case in that ablation (without the long-context clause 95%
 # and 74%; the previous rule, 8 per CU with 1024-token splits and no split at
-# 2 per CU: 85% and 19%, on a skewed batch).
+# 2 per CU: 85% and 19%, on a skewed batch).  paged_decode without a partition
+# reaches 103% on average (99% on the uniform batches, 110% on the mixed and
+# skewed ones) and 96% in the worst case.
 DECODE_WG_PER_CU = 1
 DECODE_MIN_CHUNKS = 1
 DECODE_MAX_SPLIT_CHUNKS = 4
@@ -209,8 +216,11 @@ def paged_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_le
     partition_size: tokens per split (multiple of 256); a value >= max_context_len
                   disables split-K.  None: the kernel cuts the contexts into splits
                   of about equal size; where it does not (one sequence, more than
-                  64, contexts up to 1024 tokens, less than 64 MB of K and V
-                  at max_context_len), decode_partition picks one.
+                  64, contexts up to 1024 tokens or from 2^24, less than 64 MB of K
+                  and V at max_context_len, more than 32 splits a sequence on
+                  average, one query head per kv head at D = 128 with B * H_kv
+                  between 456 and 512 and up to 8192 tokens), decode_partition
+                  picks one.
     """
     if _on_gpu(q):
         out = load_extension().plain_decode(q, k_cache, v_cache, block_tables, context_lens, max_context_len, scale,

@@ -21,13 +21,14 @@ Sections (the row schema ``attnkernels.report`` reads):
                          causal and not: the shapes of the reference's T4
                          tables (its bench/bench.py prefill sweep), so the two
                          can be read side by side
-  decode                 paged_decode (default partition, and one split) vs
+  decode                 paged_decode (splits of decode_partition's tokens, and one split) vs
                          gathering the pages then SDPA, and SDPA on a cache
                          that is already contiguous: Llama-3-8B's attention
                          layer (32 query heads, 8 kv heads, D=128, 16-token pages)
-  decode_heads           paged_decode over head-group sizes 1-8 and D 64/128
+  decode_heads           paged_decode over head-group sizes 1-8 and D 64/128, with
+                         those splits and as it chooses them itself (paged_default)
   split_ablation         every power-of-two partition from 256 tokens to one
-                         split, uniform batches
+                         split, and paged_default, uniform batches
   split_ablation_ragged  the same over batches of mixed context lengths
   ragged                 one mixed-length batch, all decode implementations
   input_activity         the headline prefill shapes and an 8192^3 fp16 GEMM on
@@ -186,6 +187,8 @@ def decode_case(section, lens, impl_names, status, partition=None, hq=LAYER["hq"
     if "paged_split" in impl_names:
         impls["paged_split"] = lambda: ak.paged_decode(q, kc, vc, tables, clens, max_ctx, partition_size=part)
         per_impl["paged_split"] = dict(partition=part, splits=-(-max_ctx // part))
+    if "paged_default" in impl_names:  # no partition given: balanced splits where they serve, else decode_partition's
+        impls["paged_default"] = lambda: ak.paged_decode(q, kc, vc, tables, clens, max_ctx)
     if "paged_nosplit" in impl_names:
         one = -(-max_ctx // ak.CHUNK) * ak.CHUNK
         impls["paged_nosplit"] = lambda: ak.paged_decode(q, kc, vc, tables, clens, max_ctx, partition_size=one)
@@ -239,8 +242,8 @@ def decode_head_builders(quick, status, max_kv_gb):
     for d in (64, 128):
         for g in (1, 2, 4, 8):
             hkv = 8
-            yield lambda d=d, g=g, hkv=hkv: decode_case("decode_heads", [c] * B, ("paged_split",), status, hq=g * hkv,
-                                                        hkv=hkv, d=d, extra=dict(group=g))
+            yield lambda d=d, g=g, hkv=hkv: decode_case("decode_heads", [c] * B, ("paged_split", "paged_default"), status,
+                                                        hq=g * hkv, hkv=hkv, d=d, extra=dict(group=g))
 
 
 def partitions_up_to(max_ctx):
@@ -251,6 +254,11 @@ def partitions_up_to(max_ctx):
         if p >= max_ctx:
             return out
         p *= 2
+
+
+def ablation_impls(partition):
+    """paged_default beside the first partition only."""
+    return ("paged_split", "paged_default") if partition == ak.CHUNK else ("paged_split",)
 
 
 def mixed_lengths(batch, lo, hi, seed):
@@ -282,7 +290,7 @@ def ablation_builders(quick, status, max_kv_gb):
             if kv_gb([c] * B, hkv) > max_kv_gb:
                 continue
             for p in partitions_up_to(c):
-                yield lambda B=B, c=c, p=p, hq=hq, hkv=hkv: decode_case("split_ablation", [c] * B, ("paged_split",),
+                yield lambda B=B, c=c, p=p, hq=hq, hkv=hkv: decode_case("split_ablation", [c] * B, ablation_impls(p),
                                                                         status, partition=p, hq=hq, hkv=hkv)
     for (hq, hkv), shapes in mixed.items():
         for B, lo, hi, seed in shapes:
@@ -291,14 +299,14 @@ def ablation_builders(quick, status, max_kv_gb):
                 continue
             for p in partitions_up_to(max(lens)):
                 yield lambda lens=lens, p=p, hq=hq, hkv=hkv: decode_case(
-                    "split_ablation_ragged", lens, ("paged_split",), status, partition=p, hq=hq, hkv=hkv,
+                    "split_ablation_ragged", lens, ablation_impls(p), status, partition=p, hq=hq, hkv=hkv,
                     extra=dict(ctx_lens=lens))
     for (hq, hkv), shapes in skewed.items():
         for B, long, short_hi, seed in shapes:
             lens = [long] + mixed_lengths(B - 1, 1, short_hi, seed)
             for p in partitions_up_to(long):
                 yield lambda lens=lens, p=p, hq=hq, hkv=hkv: decode_case(
-                    "split_ablation_ragged", lens, ("paged_split",), status, partition=p, hq=hq, hkv=hkv,
+                    "split_ablation_ragged", lens, ablation_impls(p), status, partition=p, hq=hq, hkv=hkv,
                     extra=dict(ctx_lens=lens))
 
 

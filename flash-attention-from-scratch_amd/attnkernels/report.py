@@ -93,7 +93,7 @@ def worst_error_table(rows):
 def head_group_error_table(rows):
     """Max-abs error against fp32 per head group: the grouped-query kernels
     (fp16 P) and the one-head kernel (fp32 P) on the same queries and K/V."""
-    sel = sorted((r for r in rows if r["section"] == "decode_heads" and "max_abs_err" in r),
+    sel = sorted((r for r in rows if r["section"] == "decode_heads" and r["impl"] == "paged_split" and "max_abs_err" in r),
                  key=lambda r: (r["head_dim"], r.get("group", 1)))
     body = [[r["head_dim"], r.get("group", 1), f"{r['batch']} x {r['ctx']}", f"{r['max_abs_err']:.2e}",
              f"{r['max_abs_err_one_head_path']:.2e}" if "max_abs_err_one_head_path" in r else "(the same kernel)"]
@@ -117,9 +117,9 @@ def head_group_table(rows):
     sel = [r for r in rows if r["section"] == "decode_heads"]
     if not sel:
         return ""
-    body = [[r["head_dim"], r["group"], r["heads"], r["kv_heads"], r["batch"], r["ctx"], r.get("partition", "-"),
+    body = [[r["head_dim"], r["group"], r["heads"], r["kv_heads"], r["batch"], r["ctx"], r.get("partition", "default"),
              f"{r['ms']:.4f}", f"{r['gbs']:.0f}", f"{100 * r['gbs'] / PEAK_GBS:.1f}%"]
-            for r in sorted(sel, key=lambda r: (r["head_dim"], r["group"]))]
+            for r in sorted(sel, key=lambda r: (r["head_dim"], r["group"], "partition" not in r))]
     return _table(["D", "G", "Hq", "Hkv", "B", "ctx", "P", "ms", "GB/s", "% HBM"], body)
 
 
@@ -157,10 +157,13 @@ def ablation_table(rows, section="split_ablation"):
         by_case[(r.get("heads", 32), r.get("kv_heads", 8), r["batch"], r["ctx"])].append(r)
     body = []
     for (hq, hkv, b, c), rs in sorted(by_case.items()):
-        best = max(rs, key=lambda r: r["gbs"])
-        curve = ", ".join(f"{r['partition']}:{r['gbs']:.0f}" for r in sorted(rs, key=lambda r: r["partition"]))
-        body.append([f"{hq}/{hkv}", b, c, best["partition"], f"{best['gbs']:.0f}", curve])
-    return _table(["Hq/Hkv", "B", "ctx", "best P", "best GB/s", "P:GB/s"], body)
+        default = next((r for r in rs if r["impl"] == "paged_default"), None)
+        fixed = sorted((r for r in rs if r is not default), key=lambda r: r["partition"])
+        best = max(fixed, key=lambda r: r["gbs"])
+        curve = ", ".join(f"{r['partition']}:{r['gbs']:.0f}" for r in fixed)
+        body.append([f"{hq}/{hkv}", b, c, best["partition"], f"{best['gbs']:.0f}", curve] +
+                    ([f"{default['gbs']:.0f} ({100 * default['gbs'] / best['gbs']:.0f}%)"] if default else ["-"]))
+    return _table(["Hq/Hkv", "B", "ctx", "best P", "best GB/s", "P:GB/s", "no P given (of best P)"], body)
 
 
 def activity_table(rows):

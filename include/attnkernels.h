@@ -143,11 +143,12 @@ int ak_paged_decode_fused(const void *q, const void *k_cache, const void *v_cach
  * No counterpart in the reference (its splits are `partition` tokens each,
  * attnkernels/csrc/paged_decode.cu:73-77).  The size function returns the bytes
  * of the workspace on the current device, or 0 for sizes that fixed splits
- * serve (one sequence, more than 64, max_context_len up to 1024, less than 64
- * MB of K and V at max_context_len, so few sequences and kv heads that each
- * would get more than 32 splits, invalid sizes): the call is then refused with
- * AK_ERR_UNSUPPORTED.  `partition` only
- * bounds the tokens read of a sequence, as in ak_paged_decode: those below the
+ * serve: one sequence, more than 64, max_context_len up to 1024 or from 2^24,
+ * less than 64 MB of K and V at max_context_len, so few sequences and kv heads
+ * that each would get more than 32 splits on average, with one query head per kv
+ * head at head_dim 128 and up to 8192 tokens a batch that times the kv heads is
+ * within an eighth of two per compute unit, and invalid sizes.  The call is then
+ * refused with AK_ERR_UNSUPPORTED.  `partition` only bounds the tokens read of a sequence, as in ak_paged_decode: those below the
  * smallest multiple of it >= max_context_len.  counters is required.  Arguments,
  * results and errors are otherwise those of ak_paged_decode_fused. */
 size_t ak_paged_decode_balanced_workspace_size(int64_t batch, int64_t num_heads, int64_t num_kv_heads,

@@ -15,7 +15,7 @@ src = Path(sys.argv[1]) if len(sys.argv) > 1 else root / "results" / "mi355x.jso
 data = json.loads(src.read_text())
 cases = defaultdict(list)
 for r in data["results"]:
-    if r["section"] in ("split_ablation", "split_ablation_ragged"):
+    if r["section"] in ("split_ablation", "split_ablation_ragged") and r["impl"] == "paged_split":
         cases[(r["batch"], r["heads"], r["kv_heads"], r["ctx"], r["section"])].append(r)
 rows = []
 for (b, hq, hkv, ctx, sec), rs in sorted(cases.items()):
